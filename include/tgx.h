@@ -67,6 +67,12 @@ int tgx_destination_index(const void* row_ptr_dev, int idx_bits, int64_t n_rows,
                           int64_t n_edges, void* out_dev, int out_bits,
                           void* stream);
 
+/* bad_dev[0] = 1 when some index lies outside [0, limit), else unchanged (the
+ * caller clears it): the range checks of Graph.from_coo (interop/torch/
+ * graph.py:210-218) in one pass over the array. */
+int tgx_index_range(const void* idx_dev, int idx_bits, int64_t n, int64_t limit,
+                    int32_t* bad_dev, void* stream);
+
 /* Workspace bytes needed by tgx_csr_transpose. */
 int tgx_csr_transpose_workspace(int64_t n_dst, int64_t n_src, int64_t n_edges,
                                 size_t* bytes);
@@ -100,6 +106,8 @@ int tgx_coo_to_csr_workspace(int64_t n_src, int64_t n_dst, int64_t n_edges,
  *   col_dev     [n_edges] in src's width (src_bits): src in stable dst order
  *   perm_dev    [n_edges] int32: argsort(dst, stable=True); may be NULL
  * Every dst must lie in [0, n_dst).  Supports n_edges, n_dst < 2^31.
+ * n_src > 0 says that every src lies in [0, n_src): 64-bit sources below
+ * 2^31 then move as 32-bit values; 0 says nothing about them.
  * Deterministic: output is bit-identical across runs. */
 int tgx_coo_to_csr(const void* src_dev, int src_bits, const void* dst_dev,
                    int dst_bits, int64_t n_src, int64_t n_dst, int64_t n_edges,

@@ -4,11 +4,14 @@ CPU oracle.  Integer outputs: bit-exact, including the output dtypes the
 reference constructors produce (row_ptr in dst's dtype, col_idx in src's).
 """
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 import tiga as tg
+from tiga import _native
 from oracle import ref
 
 pytestmark = pytest.mark.gpu
@@ -119,3 +122,72 @@ def test_builders_do_not_use_torch_sorting(monkeypatch):
     g.destination_index()
     g.transpose()
     tg.Graph.cu_seqlens(torch.tensor([0, 7, 20], device=DEV), causal=False).resolve_csr()
+
+
+@pytest.mark.parametrize("n_rows,n_edges", [
+    (1, 5),               # a key of no bits
+    (2, 8191),            # one tile less one key
+    (64, 8192),           # a full tile, a full 6-bit digit
+    (65, 8193),           # a second tile of one key, a 7-bit digit
+    (2048, 20_000),       # the widest single pass
+    (2049, 64 * 8192 + 1),  # two passes, a second count segment
+    (1 << 22, 30_000),    # two widest passes, most rows empty
+    ((1 << 22) + 1, 30_000),  # three passes
+])
+@pytest.mark.parametrize("src_bits,dst_bits,n_src_known", [
+    (64, 64, True), (64, 32, False), (32, 64, False), (32, 32, True)])
+def test_coo_sort_at_tile_and_digit_edges(n_rows, n_edges, src_bits, dst_bits, n_src_known):
+    """The radix sort against a stable argsort, bit for bit: sources as the
+    sort's payload (32-bit ones, and 64-bit ones known to be in range) or
+    gathered through the permutation; the permutation beside either."""
+    print(f"coo sort rows={n_rows} edges={n_edges} {src_bits}/{dst_bits}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(n_edges)
+    ints = {32: torch.int32, 64: torch.int64}
+    skew = torch.rand(n_edges, device=DEV, generator=g, dtype=torch.float64) ** 3
+    dst = (skew * n_rows).to(torch.int64).clamp_(max=n_rows - 1).to(ints[dst_bits])
+    n_src = 2**31 - 1
+    src = torch.randint(0, n_src, (n_edges,), device=DEV, generator=g).to(ints[src_bits])
+    order = torch.argsort(dst, stable=True)
+    want_ptr = torch.zeros(n_rows + 1, dtype=torch.int64, device=DEV)
+    want_ptr[1:] = torch.cumsum(torch.bincount(dst.long(), minlength=n_rows), 0)
+    row_ptr = torch.empty(n_rows + 1, dtype=dst.dtype, device=DEV)
+    col = torch.empty_like(src)
+    perm = torch.empty(n_edges, dtype=torch.int32, device=DEV)
+    ws_bytes = ctypes.c_size_t()
+    known = n_src if n_src_known else 0
+    _native.call("tgx_coo_to_csr_workspace", known, n_rows, n_edges, ctypes.byref(ws_bytes))
+    ws = torch.empty(ws_bytes.value, dtype=torch.uint8, device=DEV)
+    for want_perm in (True, False):
+        _native.call("tgx_coo_to_csr", src.data_ptr(), src_bits, dst.data_ptr(), dst_bits, known,
+                     n_rows, n_edges, row_ptr.data_ptr(), col.data_ptr(),
+                     perm.data_ptr() if want_perm else None, ws.data_ptr(), ws_bytes.value,
+                     _native.stream_of(dst))
+        assert torch.equal(row_ptr.long(), want_ptr)
+        assert torch.equal(col, src[order])
+        if want_perm:
+            assert torch.equal(perm.long(), order)
+    # The transpose of the CSR just built: row ids beside the permutation.
+    graph = tg.Graph.from_csr(row_ptr, (col.long() % 5000).to(row_ptr.dtype), num_src=5000)
+    t = graph._transposed()
+    t_order = torch.argsort(graph._col_idx, stable=True)
+    rows = torch.repeat_interleave(torch.arange(n_rows, device=DEV), want_ptr.diff())
+    assert torch.equal(graph.destination_index(), rows)
+    assert torch.equal(t.perm.long(), t_order) and torch.equal(t.col_t.long(), rows[t_order])
+    assert torch.equal(t.inv_perm[t.perm.long()].long(), torch.arange(n_edges, device=DEV))
+    tr_ptr, tr_col = graph.transpose().resolve_csr()
+    assert torch.equal(tr_ptr, t.row_ptr_t.to(tr_ptr.dtype)) and torch.equal(tr_col, t.col_t.to(
+        tr_col.dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+def test_from_coo_range_checks_and_strided_edge_lists(dtype):
+    print("from_coo range checks", flush=True)
+    pairs = torch.tensor([[0, 3], [2, 1], [4, 3], [1, 0]], dtype=dtype, device=DEV)
+    graph = tg.Graph.from_coo(pairs[:, 0], pairs[:, 1], num_src=5, num_dst=4)
+    row_ptr, col = graph.resolve_csr()
+    assert row_ptr.tolist() == [0, 1, 2, 2, 4] and col.tolist() == [1, 2, 0, 4]
+    for src, dst, name in (([0, 5], [0, 1], "src"), ([0, -1], [0, 1], "src"),
+                           ([0, 4], [0, 4], "dst"), ([0, 4], [-1, 0], "dst")):
+        with pytest.raises(ValueError, match=f"{name} contains an out-of-range"):
+            tg.Graph.from_coo(torch.tensor(src, dtype=dtype, device=DEV),
+                              torch.tensor(dst, dtype=dtype, device=DEV), num_src=5, num_dst=4)

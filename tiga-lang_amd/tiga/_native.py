@@ -61,6 +61,7 @@ ABI_VERSION = 13
 _SIGNATURES: dict[str, list] = {
     "tgx_abi_version": [],
     "tgx_destination_index": [c_vp, c_int, c_i64, c_i64, c_vp, c_int, c_vp],
+    "tgx_index_range": [c_vp, c_int, c_i64, c_i64, c_vp, c_vp],
     "tgx_csr_transpose_workspace": [c_i64, c_i64, c_i64, P(c_size)],
     "tgx_csr_transpose": [c_vp, c_vp, c_int, c_i64, c_i64, c_i64, c_vp, c_vp, c_vp,
                           c_vp, c_vp, c_size, c_vp],

@@ -134,18 +134,32 @@ def _native_builder_ok(t: torch.Tensor, n_edges: int, n_rows: int) -> bool:
     return t.is_cuda and n_edges < 2**31 and n_rows < 2**31 - 1
 
 
-def build_coo_csr(src: torch.Tensor, dst: torch.Tensor, num_dst: int):
+def _indices_out_of_range(*checks) -> list[bool]:
+    """Whether each (index tensor, limit) holds a value outside [0, limit):
+    one pass over each GPU tensor and one synchronisation for all of them."""
+    device = checks[0][0].device
+    bad = torch.zeros(len(checks), dtype=torch.int32, device=device)
+    for k, (t, limit) in enumerate(checks):
+        t = t.contiguous()
+        _native.call("tgx_index_range", t.data_ptr(), _native.idx_bits(t), t.numel(), limit,
+                     bad.data_ptr() + 4 * k, _native.stream_of(t))
+    return [b != 0 for b in bad.tolist()]
+
+
+def build_coo_csr(src: torch.Tensor, dst: torch.Tensor, num_dst: int, num_src: int = 0):
     """(row_ptr in dst's dtype, col_idx in src's dtype) for ``from_coo``:
-    stable sort of the edges by destination (reference graph.py:219-227)."""
+    stable sort of the edges by destination (reference graph.py:219-227).
+    num_src > 0: every source is known to lie in [0, num_src)."""
+    src, dst = src.contiguous(), dst.contiguous()
     device = dst.device
     E = src.numel()
     row_ptr = torch.empty(num_dst + 1, dtype=dst.dtype, device=device)
     col = torch.empty(max(E, 1), dtype=src.dtype, device=device)
     ws_bytes = ctypes.c_size_t()
-    _native.call("tgx_coo_to_csr_workspace", 0, num_dst, E, ctypes.byref(ws_bytes))
+    _native.call("tgx_coo_to_csr_workspace", num_src, num_dst, E, ctypes.byref(ws_bytes))
     ws = torch.empty(max(ws_bytes.value, 1), dtype=torch.uint8, device=device)
     _native.call("tgx_coo_to_csr", _native.ptr(src), _native.idx_bits(src), _native.ptr(dst),
-                 _native.idx_bits(dst), 0, num_dst, E, row_ptr.data_ptr(), col.data_ptr(),
+                 _native.idx_bits(dst), num_src, num_dst, E, row_ptr.data_ptr(), col.data_ptr(),
                  None, ws.data_ptr(), ws_bytes.value, _native.stream_of(dst))
     return row_ptr, col[:E]
 
@@ -303,13 +317,26 @@ class Graph:
             raise ValueError("num_src must be a non-negative integer")
         if not isinstance(num_dst, int) or num_dst < 0:
             raise ValueError("num_dst must be a non-negative integer")
+        return cls._from_coo(src, dst, num_src, num_dst)
+
+    @classmethod
+    def _from_coo(cls, src, dst, num_src: int, num_dst: int, src_known: bool = False) -> "Graph":
+        """from_coo on checked shapes and counts; src_known: every source is
+        in range by construction (the row ids of a transpose)."""
         if src.numel():
-            if int(src.min().item()) < 0 or int(src.max().item()) >= num_src:
+            if src.is_cuda:
+                *src_bad, dst_bad = _indices_out_of_range(
+                    *(() if src_known else ((src, num_src),)), (dst, num_dst))
+                src_bad = any(src_bad)
+            else:
+                src_bad = int(src.min().item()) < 0 or int(src.max().item()) >= num_src
+                dst_bad = int(dst.min().item()) < 0 or int(dst.max().item()) >= num_dst
+            if src_bad:
                 raise ValueError("src contains an out-of-range source index")
-            if int(dst.min().item()) < 0 or int(dst.max().item()) >= num_dst:
+            if dst_bad:
                 raise ValueError("dst contains an out-of-range destination index")
         if _native_builder_ok(dst, src.numel(), num_dst):
-            row_ptr, col_idx = build_coo_csr(src, dst, num_dst)
+            row_ptr, col_idx = build_coo_csr(src, dst, num_dst, num_src)
         else:
             order = torch.argsort(dst, stable=True)
             col_idx = src[order]
@@ -497,15 +524,28 @@ class Graph:
 
     def transpose(self) -> "Graph":
         row_ptr, col_idx = self.resolve_csr()
-        destination = self.destination_index(row_ptr)
-        return type(self).from_coo(destination.to(col_idx.dtype), col_idx,
-                                   num_src=self._schema.num_dst, num_dst=self._schema.num_src)
+        cached = self._destination_index_cache if self._row_ptr is row_ptr else None
+        destination = (self._destination_rows(row_ptr, col_idx.dtype) if cached is None
+                       else cached.to(col_idx.dtype))
+        if destination.dtype == torch.int64 and self._row_ptr is row_ptr:
+            self._destination_index_cache = destination
+        if destination.shape != col_idx.shape:
+            raise ValueError("src and dst must have identical shapes")
+        return self._from_coo(destination, col_idx, self._schema.num_dst, self._schema.num_src,
+                              src_known=True)
 
     def destination_index(self, row_ptr: torch.Tensor | None = None) -> torch.Tensor:
         if row_ptr is None and self._destination_index_cache is not None:
             return self._destination_index_cache
         if row_ptr is None:
             row_ptr, _ = self.resolve_csr()
+        dst = self._destination_rows(row_ptr, torch.int64)
+        if self._row_ptr is row_ptr:
+            self._destination_index_cache = dst
+        return dst
+
+    def _destination_rows(self, row_ptr: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+        """The destination row of every edge, in `dtype`."""
         native = False
         if row_ptr.is_cuda and row_ptr.numel() == self._schema.num_dst + 1 > 1:
             # One sync: the edge count, and whether row_ptr is well formed
@@ -518,17 +558,15 @@ class Graph:
             native = bool(stats[1]) and bool(stats[2]) and _native_builder_ok(
                 row_ptr, n_edges, self._schema.num_dst)
         if native:
-            dst = torch.empty(n_edges, dtype=torch.int64, device=row_ptr.device)
+            row_ptr = row_ptr.contiguous()
+            dst = torch.empty(n_edges, dtype=dtype, device=row_ptr.device)
             _native.call("tgx_destination_index", _native.ptr(row_ptr),
                          _native.idx_bits(row_ptr), self._schema.num_dst, n_edges,
-                         _native.ptr(dst), 64, _native.stream_of(row_ptr))
-        else:
-            degree = row_ptr[1:] - row_ptr[:-1]
-            dst = torch.repeat_interleave(
-                torch.arange(self._schema.num_dst, device=row_ptr.device), degree)
-        if self._row_ptr is row_ptr:
-            self._destination_index_cache = dst
-        return dst
+                         _native.ptr(dst), _native.idx_bits(dst), _native.stream_of(row_ptr))
+            return dst
+        degree = row_ptr[1:] - row_ptr[:-1]
+        return torch.repeat_interleave(
+            torch.arange(self._schema.num_dst, device=row_ptr.device), degree).to(dtype)
 
     def _degree_stats(self) -> tuple[int, int, int]:
         """(min, max, sum) of the destination-row degrees: closed forms for
