@@ -219,8 +219,7 @@ int tgx_plan_reference_buckets(int64_t n_rows, int64_t max_degree,
  *   col_dev NULL: the columns are the edge ids, i.e. x_dev [n_edges, F] is a
  *   per-edge field summed per destination row (n_src = n_edges < 2^31; the
  *   per-edge input gradients of an edge network reduce this way).
- * F may be any positive width; widths that are multiples of 4 with
- * F*4 <= 1024 bytes take the vectorised path. */
+ * F may be any positive width; rows need the alignment of their elements. */
 int tgx_csr_sum_fwd(const void* row_ptr_dev, const void* col_dev, int idx_bits,
                     const tgx_row_plan* plan, const void* x_dev,
                     const float* w_dev, void* out_dev, int64_t n_dst,
@@ -243,6 +242,19 @@ int tgx_csr_sum_bwd(const int32_t* row_ptr_t_dev, const int32_t* col_t_dev,
                     const void* dout_dev, void* dx_dev, float* dw_dev,
                     int64_t n_dst, int64_t n_src, int64_t F, int dtype,
                     float* partial_dev, void* stream);
+
+/* tgx_csr_sum_bwd with a workspace: rows wider than a feature tile (64 lanes of
+ * 16 bytes) then get dw from the sum's own pass, a partial sum per tile and
+ * edge, where tgx_csr_sum_bwd runs a pass of its own for it.  The workspace is
+ * 0 bytes where one tile covers F; n_edges = the relation's edges. */
+int tgx_csr_sum_bwd_workspace(int64_t n_edges, int64_t F, int dtype, size_t* bytes);
+int tgx_csr_sum_bwd_ws(const int32_t* row_ptr_t_dev, const int32_t* col_t_dev,
+                       const int32_t* perm_dev, const tgx_row_plan* plan_t,
+                       const void* x_dev, const float* w_dev,
+                       const void* dout_dev, void* dx_dev, float* dw_dev,
+                       int64_t n_dst, int64_t n_src, int64_t n_edges, int64_t F,
+                       int dtype, float* partial_dev, void* workspace_dev,
+                       size_t workspace_bytes, void* stream);
 
 /* Per-edge dot products in edge order over the destination-row CSR:
  *   dw[e] = <dout[row(e), :], x[col[e], :]>,  e = 0 .. n_edges-1

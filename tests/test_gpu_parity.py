@@ -236,6 +236,48 @@ def test_sum_of_edge_field_per_row(F_, idx):
     assert rel_err(out.cpu(), ref.sum_fwd(rp, np.arange(E), x)) <= RTOL32
 
 
+# Widths at the edges of a lane's values (4 fp32, 8 16-bit) and of the lane
+# groups, rows aligned to their elements only; tables one L2 holds whole (900
+# source rows of few values), a column tile at a time (9,000 rows of 260 or
+# more values), and not at all (70,000 destination rows: the backward's).
+@pytest.mark.parametrize("n_dst,n_src,F_", [
+    *[(1500, 900, f) for f in (1, 3, 4, 5, 7, 8, 9, 31, 33, 63, 65, 127, 129, 255, 257)],
+    (9000, 9000, 260), (9000, 8000, 301), (6000, 40000, 517), (5000, 3000, 1030),
+    (70000, 3000, 301)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_sum_width_and_tile_edges(n_dst, n_src, F_, dtype):
+    """fp32 sums against float64: fp32 outputs within their rounding (1e-5 of
+    the largest), 16-bit ones within one rounding of the element type."""
+    print(f"sum widths {n_dst}x{n_src} F={F_} {dtype}", flush=True)
+    rp, col = skewed_csr(F_, n_dst, n_src, mean_deg=4, hubs=(1300, 200, 129, 40), hot_src=3,
+                         hot_frac=0.03)
+    E = col.size
+    row_ptr, cols = to_dev(rp, torch.int64), to_dev(col, torch.int64)
+    g = torch.Generator(device=DEV).manual_seed(F_)
+    x = torch.randn(n_src, F_, device=DEV, generator=g).to(dtype)
+    w = torch.rand(E, device=DEV, generator=g)
+    dout = torch.randn(n_dst, F_, device=DEV, generator=g).to(dtype)
+    graph = tg.Graph.from_csr(row_ptr, cols, num_src=n_src)
+    rows = graph.destination_index()
+    x64, w64, d64 = x.double(), w.double()[:, None], dout.double()
+    want = torch.zeros(n_dst, F_, dtype=torch.float64, device=DEV).index_add_(
+        0, rows, w64 * x64[cols])
+    want_dx = torch.zeros_like(x64).index_add_(0, cols, w64 * d64[rows])
+    want_dw = (x64[cols] * d64[rows]).sum(1)
+    from tiga._ops import CsrSumFunction
+
+    eps = {torch.float32: 1e-5, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -10}[dtype]
+    xg, wg = x.clone().requires_grad_(True), w.clone().requires_grad_(True)
+    out = CsrSumFunction.apply(xg, wg, graph)
+    dx, dw = torch.autograd.grad(out, (xg, wg), dout, retain_graph=True)
+    (dw_only,) = torch.autograd.grad(out, (wg,), dout, retain_graph=True)
+    (dx_only,) = torch.autograd.grad(out, (xg,), dout)
+    assert rel_err(out.detach().double().cpu(), want.cpu()) <= eps
+    assert rel_err(dx.double().cpu(), want_dx.cpu()) <= eps
+    assert rel_err(dw.double().cpu(), want_dw.cpu()) <= RTOL32
+    assert torch.equal(dx, dx_only) and torch.equal(dw, dw_only)
+
+
 # ---- GAT additive ----------------------------------------------------------
 
 class GAT(tg.MessagePassing):

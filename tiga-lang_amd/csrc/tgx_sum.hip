@@ -1,17 +1,33 @@
 // Sum reducer over a destination-row CSR:  out[i, :] = sum_e w[e] * x[col[e], :]
 //
-// Layout: a gathered row of F fp32 features is split into feature tiles of
-// G*VEC floats; G lanes hold one tile of one edge, VEC floats per lane
-// (16-byte loads when VEC == 4), so one wave keeps 64/G edges in flight per
-// vector load and U such loads per lane before consuming them.  The edge
-// groups are folded at the end of the row with cross-lane adds.
+// Layout: a gathered row of F features is split into feature tiles of G*VEC
+// values; G lanes hold one tile of one edge, 16 bytes per lane (VEC = 4 fp32
+// or 8 16-bit values; fewer only where F is smaller), so one wave keeps 64/G
+// edges in flight per vector load and U such loads per lane before consuming
+// them.  Any F >= VEC takes the 16-byte loads: the last lane of a row moves
+// back to the row's last VEC values where F is no multiple of VEC (it repeats
+// values of its neighbour, to the bit), and rows need only the alignment of
+// their elements.  The edge groups are folded at the end of the row with
+// cross-lane adds.
 //
 // The same kernel is the backward's dx pass: run over the transposed CSR with
 // x := dout and the weight fetched through the transpose permutation, it
 // computes dx[j] = sum_{e'} w[perm[e']] * dout[col_t[e']] with no atomics.  With
 // `self_x` set it also produces dw[perm[e']] = <dout[col_t[e']], x[j]> from the
 // row it already holds.
+//
+// What bounds it: the L2s fetch about 55 G lines a second from beyond
+// (Infinity Cache or HBM alike, 64 or 128 bytes of a line alike), 7 TB/s of
+// whole lines, and a random row costs the lines it touches.  100,000 rows of
+// 16 neighbours, 64 floats: 57 us for 3.2 M lines; 200,000 rows of 12
+// neighbours, 100 bf16: 178 us with one row per wave and 8-byte loads, 116 us
+// for 6.1 M lines now.  (Column tiles of 128 bytes, each XCD's L2 holding one
+// of a 20,000 x 500 table, measured slower than whole rows, 60 against 52 us:
+// the edges are then walked 16 times.)
 #include <hip/hip_runtime.h>
+
+#include <climits>
+#include <type_traits>
 
 #include "tgx_device.h"
 #include "tgx_host.h"
@@ -21,53 +37,107 @@
 namespace tgx {
 namespace {
 
-// Element storage of the feature tables (x, out, dout, dx); weights and the
-// split-row partials are always fp32, and so is every sum.
+// VEC consecutive features of one lane: Raw as loaded, widened to fp32 as it
+// is consumed.  Weights and the split-row partials are always fp32, and so is
+// every sum.  (The vector types claim an element's alignment only; gfx950
+// loads and stores 16 bytes at any address.)
+typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x4_u __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x2_u __attribute__((ext_vector_type(2), aligned(2)));
+
 template <int DT>
 struct Elem;
 template <>
 struct Elem<TGX_DTYPE_F32> {
   typedef float S;
-  static __device__ __forceinline__ f32x4 load4(const S* p) {
-    return *reinterpret_cast<const f32x4*>(p);
-  }
-  static __device__ __forceinline__ void store4(S* p, f32x4 v) {
-    *reinterpret_cast<f32x4*>(p) = v;
-  }
   static __device__ __forceinline__ float load1(const S* p) { return *p; }
   static __device__ __forceinline__ void store1(S* p, float v) { *p = v; }
 };
 template <>
 struct Elem<TGX_DTYPE_BF16> {
   typedef uint16_t S;
-  static __device__ __forceinline__ f32x4 load4(const S* p) {
-    const uint2 w = *reinterpret_cast<const uint2*>(p);
-    return f32x4{bf16_lo(w.x), bf16_hi(w.x), bf16_lo(w.y), bf16_hi(w.y)};
-  }
-  static __device__ __forceinline__ void store4(S* p, f32x4 v) {
-    *reinterpret_cast<uint2*>(p) = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-  }
   static __device__ __forceinline__ float load1(const S* p) { return bf16_lo(*p); }
   static __device__ __forceinline__ void store1(S* p, float v) {
     *p = static_cast<uint16_t>(f32_to_bf16_bits(v));
   }
+  static __device__ __forceinline__ void widen2(uint32_t w, float* f) {
+    f[0] = bf16_lo(w);
+    f[1] = bf16_hi(w);
+  }
+  static __device__ __forceinline__ uint32_t pack2(float a, float b) { return pack_bf16x2(a, b); }
 };
 template <>
 struct Elem<TGX_DTYPE_F16> {
   typedef _Float16 S;
-  typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-  static __device__ __forceinline__ f32x4 load4(const S* p) {
-    const h4 h = *reinterpret_cast<const h4*>(p);
-    return f32x4{static_cast<float>(h[0]), static_cast<float>(h[1]), static_cast<float>(h[2]),
-                 static_cast<float>(h[3])};
-  }
-  static __device__ __forceinline__ void store4(S* p, f32x4 v) {
-    *reinterpret_cast<h4*>(p) = h4{static_cast<_Float16>(v[0]), static_cast<_Float16>(v[1]),
-                                   static_cast<_Float16>(v[2]), static_cast<_Float16>(v[3])};
-  }
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
   static __device__ __forceinline__ float load1(const S* p) { return static_cast<float>(*p); }
   static __device__ __forceinline__ void store1(S* p, float v) { *p = static_cast<_Float16>(v); }
+  static __device__ __forceinline__ void widen2(uint32_t w, float* f) {
+    const h2 h = __builtin_bit_cast(h2, w);
+    f[0] = static_cast<float>(h[0]);
+    f[1] = static_cast<float>(h[1]);
+  }
+  static __device__ __forceinline__ uint32_t pack2(float a, float b) {
+    return __builtin_bit_cast(uint32_t, h2{static_cast<_Float16>(a), static_cast<_Float16>(b)});
+  }
 };
+
+template <int VEC, int DT>
+struct Vec {   // 16-bit elements, VEC = 4 or 8
+  typedef std::conditional_t<VEC == 8, u32x4_u, u32x2_u> Raw;
+  typedef typename Elem<DT>::S S;
+  static __device__ __forceinline__ Raw load(const S* p) {
+    return *reinterpret_cast<const Raw*>(p);
+  }
+  static __device__ __forceinline__ void widen(Raw r, float (&f)[VEC]) {
+#pragma unroll
+    for (int k = 0; k < VEC / 2; ++k) Elem<DT>::widen2(r[k], f + 2 * k);
+  }
+  static __device__ __forceinline__ void store(S* p, const float (&f)[VEC]) {
+    Raw r;
+#pragma unroll
+    for (int k = 0; k < VEC / 2; ++k) r[k] = Elem<DT>::pack2(f[2 * k], f[2 * k + 1]);
+    *reinterpret_cast<Raw*>(p) = r;
+  }
+};
+template <>
+struct Vec<4, TGX_DTYPE_F32> {
+  typedef f32x4_u Raw;
+  typedef float S;
+  static __device__ __forceinline__ Raw load(const S* p) {
+    return *reinterpret_cast<const Raw*>(p);
+  }
+  static __device__ __forceinline__ void widen(Raw r, float (&f)[4]) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) f[k] = r[k];
+  }
+  static __device__ __forceinline__ void store(S* p, const float (&f)[4]) {
+    *reinterpret_cast<Raw*>(p) = Raw{f[0], f[1], f[2], f[3]};
+  }
+};
+template <int DT>
+struct Vec<1, DT> {
+  typedef typename Elem<DT>::S S;
+  typedef S Raw;
+  static __device__ __forceinline__ Raw load(const S* p) { return *p; }
+  static __device__ __forceinline__ void widen(Raw r, float (&f)[1]) {
+    f[0] = Elem<DT>::load1(&r);
+  }
+  static __device__ __forceinline__ void store(S* p, const float (&f)[1]) {
+    Elem<DT>::store1(p, f[0]);
+  }
+};
+// A lane's values of a split row's fp32 partial.
+template <int VEC>
+__device__ __forceinline__ void store_partial(float* p, const float (&f)[VEC]) {
+  if constexpr (VEC == 1) {
+    p[0] = f[0];
+  } else {
+#pragma unroll
+    for (int k = 0; k < VEC; k += 4)
+      *reinterpret_cast<f32x4_u*>(p + k) = f32x4_u{f[k], f[k + 1], f[k + 2], f[k + 3]};
+  }
+}
 
 template <typename I, int DT>
 struct SumArgs {
@@ -81,80 +151,76 @@ struct SumArgs {
   S* out;                  // [rows, F]
   float* partial;          // [n_chunks, F]
   const S* self_x;         // dw: row's own features [rows, F] (null = no dw)
-  float* dw;               // dw output, written at wperm ? wperm[e] : e
+  float* dw;               // dw output, written at dwperm ? dwperm[e] : e
+  const int32_t* dwperm;
   int64_t F;
+  int64_t dw_tile;         // floats between the feature tiles' dw (dw sums of one tile each)
 };
 
-// VEC consecutive features per lane, held in fp32.
+// A lane's features of the tile: the offset of its VEC values in a row, and
+// how many of them its neighbour holds too (a moved last lane).
+struct LaneCols {
+  int64_t at;
+  int repeated;
+  bool active;
+};
+template <int VEC>
+__device__ __forceinline__ LaneCols lane_cols(int64_t first, int64_t F) {
+  LaneCols l{first, 0, first < F};
+  if constexpr (VEC > 1) {
+    l.at = first < F - VEC ? first : F - VEC;
+    l.repeated = static_cast<int>(first - l.at);
+  }
+  return l;
+}
+
+// The row's own values for dw; repeated ones count once.
 template <int VEC, int DT>
-struct Vec;
-template <int DT>
-struct Vec<4, DT> {
-  typedef f32x4 T;
-  typedef typename Elem<DT>::S S;
-  static __device__ __forceinline__ T load(const S* p) { return Elem<DT>::load4(p); }
-  static __device__ __forceinline__ void store(S* p, T v) { Elem<DT>::store4(p, v); }
-  static __device__ __forceinline__ T zero() { return f32x4{0.f, 0.f, 0.f, 0.f}; }
-  static __device__ __forceinline__ float dot(T a, T b) {
-    return a[0] * b[0] + a[1] * b[1] + a[2] * b[2] + a[3] * b[3];
-  }
-  static __device__ __forceinline__ T shfl_xor(T v, int m) {
-    return f32x4{__shfl_xor(v[0], m, 64), __shfl_xor(v[1], m, 64),
-                 __shfl_xor(v[2], m, 64), __shfl_xor(v[3], m, 64)};
-  }
-};
-template <int DT>
-struct Vec<1, DT> {
-  typedef float T;
-  typedef typename Elem<DT>::S S;
-  static __device__ __forceinline__ T load(const S* p) { return Elem<DT>::load1(p); }
-  static __device__ __forceinline__ void store(S* p, T v) { Elem<DT>::store1(p, v); }
-  static __device__ __forceinline__ T zero() { return 0.f; }
-  static __device__ __forceinline__ float dot(T a, T b) { return a * b; }
-  static __device__ __forceinline__ T shfl_xor(T v, int m) { return __shfl_xor(v, m, 64); }
-};
+__device__ __forceinline__ void load_self(const typename Elem<DT>::S* row, const LaneCols& l,
+                                          float (&self)[VEC]) {
+  Vec<VEC, DT>::widen(Vec<VEC, DT>::load(row + l.at), self);
+#pragma unroll
+  for (int k = 0; k < VEC; ++k)
+    if (k < l.repeated) self[k] = 0.f;
+}
 
-template <int G>
-__device__ __forceinline__ float group_reduce_sum(float v) {
-  // Sum over the G lanes of one edge group (aligned, contiguous).
-  return group_sum<G>(v);
+template <int VEC>
+__device__ __forceinline__ float dot(const float (&a)[VEC], const float (&b)[VEC]) {
+  float s = 0.f;
+#pragma unroll
+  for (int k = 0; k < VEC; ++k) s += a[k] * b[k];
+  return s;
 }
 
 // One whole-wave task (a row, a split-row chunk or a group of empty rows).
 template <typename I, int DT, int VEC, int G, int U>
-__device__ __forceinline__ void sum_task(const SumArgs<I, DT>& a, const Task& t) {
+__device__ __forceinline__ void sum_task(const SumArgs<I, DT>& a, const Task& t, int tile,
+                                         float* dw_stage) {
   typedef Vec<VEC, DT> V;
-  typedef typename V::T T;
   constexpr int EPW = kWave / G;  // edges per wave-wide load
   if (t.kind == kTaskNone) return;
   const int lane = lane_id();
   const int g = lane / G;
   const int c = lane % G;
   const int64_t F = a.F;
-  const int64_t fo = static_cast<int64_t>(blockIdx.y) * (G * VEC) + c * VEC;
-  const bool active = fo < F;
+  const LaneCols lc = lane_cols<VEC>(static_cast<int64_t>(tile) * (G * VEC) + c * VEC, F);
 
   if (t.kind == kTaskEmpty) {
     for (int k = 0; k < t.n_empty; ++k) {
       const int row = uniform(a.plan.rows[t.empty0 + k]);
-      if (g == 0 && active && a.out)
-        V::store(a.out + static_cast<int64_t>(row) * F + fo, V::zero());
+      const float zero[VEC] = {};
+      if (g == 0 && lc.active && a.out)
+        V::store(a.out + static_cast<int64_t>(row) * F + lc.at, zero);
     }
     return;
   }
 
-  T self = V::zero();
+  float self[VEC] = {};
   const bool want_dw = a.self_x != nullptr;
-  if (want_dw && active) self = V::load(a.self_x + static_cast<int64_t>(t.row) * F + fo);
-  // A window's dw values wait in LDS and leave with one store per lane
-  // after the window, not one store per edge group inside the gather loop
-  // (whose following gathers would share its in-order completion count).
-  // Measured on bench.py --config c1: the backward unchanged (0.109 ms), the forward, which
-  // writes no dw, 0.061 -> 0.059 ms with this kernel shape.
-  __shared__ float dw_stage[kWavesPerBlock][kWave];
-  const int wv = threadIdx.x / kWave;
+  if (want_dw && lc.active)
+    load_self<VEC, DT>(a.self_x + static_cast<int64_t>(t.row) * F, lc, self);
 
-  T acc = V::zero();
+  float acc[VEC] = {};
   for (int64_t base = t.e0; base < t.e1; base += kWave) {
     const int n = static_cast<int>(t.e1 - base < kWave ? t.e1 - base : kWave);
     int my_col = 0;
@@ -169,7 +235,7 @@ __device__ __forceinline__ void sum_task(const SumArgs<I, DT>& a, const Task& t)
       my_w = a.w ? a.w[a.wperm ? static_cast<int64_t>(my_wp) : e] : 1.f;
     }
     for (int k = 0; k < n; k += EPW * U) {
-      T v[U];
+      typename V::Raw v[U];
       float wt[U];
       int slot[U];
 #pragma unroll
@@ -178,83 +244,98 @@ __device__ __forceinline__ void sum_task(const SumArgs<I, DT>& a, const Task& t)
         const int src = slot[u] < n ? slot[u] : 0;
         const int j = __shfl(my_col, src, 64);
         wt[u] = __shfl(my_w, src, 64);
-        v[u] = (slot[u] < n && active) ? V::load(a.x + static_cast<int64_t>(j) * F + fo)
-                                       : V::zero();
+        v[u] = typename V::Raw{};
+        if (slot[u] < n && lc.active) v[u] = V::load(a.x + static_cast<int64_t>(j) * F + lc.at);
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        if (slot[u] < n) acc += wt[u] * v[u];
-      }
-      if (want_dw) {
+        float f[VEC];
+        V::widen(v[u], f);
+        if (slot[u] < n) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const float d = group_reduce_sum<G>(V::dot(v[u], self));
-          if (c == 0 && slot[u] < n) dw_stage[wv][slot[u]] = d;
+          for (int q = 0; q < VEC; ++q) acc[q] += wt[u] * f[q];
+        }
+        if (want_dw) {
+          const float d = group_sum<G>(dot(f, self));
+          if (c == 0 && slot[u] < n) dw_stage[slot[u]] = d;
         }
       }
     }
     if (want_dw) {
+      // A window's dw values wait in LDS and leave with one store per lane
+      // after the window, not one store per edge group inside the gather loop
+      // (whose following gathers would share its in-order completion count).
       // One wave's LDS accesses complete in issue order: lane e reads the
       // value another lane wrote for edge base + e.
       __builtin_amdgcn_wave_barrier();
-      if (lane < n) a.dw[a.wperm ? static_cast<int64_t>(my_wp) : base + lane] = dw_stage[wv][lane];
+      if (lane < n) {
+        const int64_t at = a.dwperm ? static_cast<int64_t>(a.wperm ? my_wp : a.dwperm[base + lane])
+                                    : base + lane;
+        a.dw[tile * a.dw_tile + at] = dw_stage[lane];
+      }
       __builtin_amdgcn_wave_barrier();
     }
   }
   // Fold the EPW edge groups (lanes with equal c).
 #pragma unroll
-  for (int m = G; m < kWave; m <<= 1) acc += V::shfl_xor(acc, m);
+  for (int m = G; m < kWave; m <<= 1)
+#pragma unroll
+    for (int q = 0; q < VEC; ++q) acc[q] += __shfl_xor(acc[q], m, 64);
   // A null out: only the per-edge dot products (dw) are wanted.
-  if (g != 0 || !active || !a.out) return;
+  if (g != 0 || !lc.active || !a.out) return;
   if (t.kind == kTaskChunk)
-    Vec<VEC, TGX_DTYPE_F32>::store(a.partial + static_cast<int64_t>(t.slot) * F + fo, acc);
+    store_partial<VEC>(a.partial + static_cast<int64_t>(t.slot) * F + lc.at, acc);
   else
-    V::store(a.out + static_cast<int64_t>(t.row) * F + fo, acc);
+    V::store(a.out + static_cast<int64_t>(t.row) * F + lc.at, acc);
 }
 
 template <typename I, int DT, int VEC, int G, int U>
 __global__ __launch_bounds__(kTaskBlock) void sum_rows_kernel(SumArgs<I, DT> a) {
-  sum_task<I, DT, VEC, G, U>(a, decode_task(a.plan, a.row_ptr, global_wave()));
+  __shared__ float dw_stage[kWavesPerBlock][kWave];
+  sum_task<I, DT, VEC, G, U>(a, decode_task(a.plan, a.row_ptr, global_wave()), blockIdx.y,
+                             dw_stage[threadIdx.x / kWave]);
 }
 
-// Narrow rows (G <= 8 lanes per edge): the wave splits into 64 / SLOT lane
+// Narrow tiles (G <= 16 lanes per edge): the wave splits into 64 / SLOT lane
 // slots of SLOT lanes, each taking P rows of the wave bin, so a wave's fixed
 // cost (task decode, the dependent row_ptr -> col -> gather chain) covers
 // (64 / SLOT) P rows, and the loads of a slot's P rows are in flight
-// together.  A slot keeps SLOT edges per row in flight (U = G loads of
-// SLOT / G edges).  The task list is
+// together.  A slot keeps U SLOT / G edges per row in flight.  The task list is
 //   [split-row chunks | row groups | empty-row groups];
-// chunks and empty groups run as whole-wave tasks.  Slot s of group w takes
-// the wave-bin rows S P w + S q + s, q < P, S = 64 / SLOT.
-template <typename I, int DT, int VEC, int G, int UC, int SLOT, int P>
+// chunks and empty groups run as whole-wave tasks, and after the group's other
+// rows so does each row of over kSlotRow edges.  Slot s of group w takes the
+// wave-bin rows S P w + S q + s, q < P, S = 64 / SLOT.
+template <int SLOT>
+constexpr int kSlotRow = 4 * SLOT;
+
+template <typename I, int DT, int VEC, int G, int UC, int SLOT, int P, int U>
 __global__ __launch_bounds__(kTaskBlock) void sum_pairs_kernel(SumArgs<I, DT> a) {
   typedef Vec<VEC, DT> V;
-  typedef typename V::T T;
   constexpr int NS = kWave / SLOT;   // slots per wave
   constexpr int EPH = SLOT / G;      // edges per slot load
-  constexpr int U = G;               // loads in flight per row: SLOT edges
+  __shared__ float dw_stage[kWavesPerBlock][P * kWave];
   const PlanView& p = a.plan;
+  const int wv = threadIdx.x / kWave;
+  float* const stage = dw_stage[wv];
   const int64_t w = global_wave();
   const int64_t n_groups = (p.n_wave + NS * P - 1) / (NS * P);
-  if (w < p.n_chunks) {
-    sum_task<I, DT, VEC, G, UC>(a, decode_task(p, a.row_ptr, w));
-    return;
-  }
   const int64_t pw = w - p.n_chunks;
-  if (pw >= n_groups) {
-    sum_task<I, DT, VEC, G, UC>(a, decode_task(p, a.row_ptr, p.n_chunks + p.n_wave + (pw - n_groups)));
+  if (pw < 0 || pw >= n_groups) {
+    sum_task<I, DT, VEC, G, UC>(
+        a, decode_task(p, a.row_ptr, pw < 0 ? w : p.n_chunks + p.n_wave + (pw - n_groups)), 0,
+        stage);
     return;
   }
   const int lane = lane_id();
   const int slot_id = lane / SLOT, hl = lane % SLOT;
   const int g = hl / G, c = hl % G;
   const int64_t F = a.F;
-  const int64_t fo = c * VEC;   // G * VEC <= F's tile: one feature tile
-  const bool active = fo < F;
+  const LaneCols lc = lane_cols<VEC>(c * VEC, F);   // (one tile)
   const bool want_dw = a.self_x != nullptr;
   int row[P], len[P];
   int64_t e0[P];
-  bool has[P];
+  bool has[P];      // rows the slots sum here
+  uint64_t late[P]; // lanes of the slots whose row runs whole-wave afterwards
   int len_max = 0;
 #pragma unroll
   for (int q = 0; q < P; ++q) {
@@ -263,20 +344,23 @@ __global__ __launch_bounds__(kTaskBlock) void sum_pairs_kernel(SumArgs<I, DT> a)
     row[q] = has[q] ? p.rows[p.n_empty + k] : 0;
     e0[q] = has[q] ? static_cast<int64_t>(a.row_ptr[row[q]]) : 0;
     len[q] = has[q] ? static_cast<int>(static_cast<int64_t>(a.row_ptr[row[q] + 1]) - e0[q]) : 0;
+    late[q] = __ballot(hl == 0 && len[q] > kSlotRow<SLOT>);
+    if (len[q] > kSlotRow<SLOT>) {
+      has[q] = false;
+      len[q] = 0;
+    }
     len_max = max(len_max, len[q]);
   }
   // Every slot loops to the longest row (wave-uniform bounds keep every
   // shuffle's source lanes active); each row masks its own tail.
 #pragma unroll
   for (int m = SLOT; m < kWave; m <<= 1) len_max = max(len_max, __shfl_xor(len_max, m, 64));
-  T self[P], acc[P];
+  len_max = uniform(len_max);
+  float self[P][VEC] = {}, acc[P][VEC] = {};
 #pragma unroll
-  for (int q = 0; q < P; ++q) {
-    self[q] = V::zero();
-    acc[q] = V::zero();
-    if (want_dw && active && has[q])
-      self[q] = V::load(a.self_x + static_cast<int64_t>(row[q]) * F + fo);
-  }
+  for (int q = 0; q < P; ++q)
+    if (want_dw && lc.active && has[q])
+      load_self<VEC, DT>(a.self_x + static_cast<int64_t>(row[q]) * F, lc, self[q]);
   for (int base = 0; base < len_max; base += SLOT) {
     int n[P], my_col[P], my_wp[P];
     float my_w[P];
@@ -295,7 +379,7 @@ __global__ __launch_bounds__(kTaskBlock) void sum_pairs_kernel(SumArgs<I, DT> a)
     }
     const int n_max = min(len_max - base, SLOT);   // wave-uniform
     for (int kk = 0; kk < n_max; kk += EPH * U) {
-      T v[P][U];
+      typename V::Raw v[P][U];
       float wt[P][U];
       int slot[U];
 #pragma unroll
@@ -307,26 +391,37 @@ __global__ __launch_bounds__(kTaskBlock) void sum_pairs_kernel(SumArgs<I, DT> a)
           const int src = SLOT * slot_id + (slot[u] < n[q] ? slot[u] : 0);
           const int j = __shfl(my_col[q], src, 64);
           wt[q][u] = __shfl(my_w[q], src, 64);
-          v[q][u] = (slot[u] < n[q] && active) ? V::load(a.x + static_cast<int64_t>(j) * F + fo)
-                                               : V::zero();
+          v[q][u] = typename V::Raw{};
+          if (slot[u] < n[q] && lc.active)
+            v[q][u] = V::load(a.x + static_cast<int64_t>(j) * F + lc.at);
         }
 #pragma unroll
       for (int q = 0; q < P; ++q)
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-          if (slot[u] < n[q]) acc[q] += wt[q][u] * v[q][u];
-      if (want_dw) {
+        for (int u = 0; u < U; ++u) {
+          float f[VEC];
+          V::widen(v[q][u], f);
+          if (slot[u] < n[q]) {
 #pragma unroll
-        for (int q = 0; q < P; ++q)
-#pragma unroll
-          for (int u = 0; u < U; ++u) {
-            const float d = group_reduce_sum<G>(V::dot(v[q][u], self[q]));
-            const int k = slot[u] < n[q] ? slot[u] : 0;
-            const int wp = __shfl(my_wp[q], SLOT * slot_id + k, 64);
-            const int64_t widx = a.wperm ? static_cast<int64_t>(wp) : e0[q] + base + k;
-            if (c == 0 && slot[u] < n[q]) a.dw[widx] = d;
+            for (int r = 0; r < VEC; ++r) acc[q][r] += wt[q][u] * f[r];
           }
-      }
+          if (want_dw) {
+            const float d = group_sum<G>(dot(f, self[q]));
+            if (c == 0 && slot[u] < n[q]) stage[q * kWave + SLOT * slot_id + slot[u]] = d;
+          }
+        }
+    }
+    if (want_dw) {
+      // (As in sum_task: dw leaves after the window, one store per lane.)
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int q = 0; q < P; ++q)
+        if (hl < n[q]) {
+          const int64_t e = e0[q] + base + hl;
+          const int64_t at = a.dwperm ? static_cast<int64_t>(a.wperm ? my_wp[q] : a.dwperm[e]) : e;
+          a.dw[at] = stage[q * kWave + lane];
+        }
+      __builtin_amdgcn_wave_barrier();
     }
   }
   // Fold each row's edge groups (lanes with equal c; masks below SLOT stay
@@ -334,10 +429,18 @@ __global__ __launch_bounds__(kTaskBlock) void sum_pairs_kernel(SumArgs<I, DT> a)
 #pragma unroll
   for (int q = 0; q < P; ++q) {
 #pragma unroll
-    for (int m = G; m < SLOT; m <<= 1) acc[q] += V::shfl_xor(acc[q], m);
-    if (g == 0 && active && has[q] && a.out)
-      V::store(a.out + static_cast<int64_t>(row[q]) * F + fo, acc[q]);
+    for (int m = G; m < SLOT; m <<= 1)
+#pragma unroll
+      for (int r = 0; r < VEC; ++r) acc[q][r] += __shfl_xor(acc[q][r], m, 64);
+    if (g == 0 && lc.active && has[q] && a.out)
+      V::store(a.out + static_cast<int64_t>(row[q]) * F + lc.at, acc[q]);
   }
+#pragma unroll
+  for (int q = 0; q < P; ++q)
+    for (uint64_t m = late[q]; m; m &= m - 1) {
+      const int64_t k = NS * P * pw + NS * q + (__ffsll(static_cast<long long>(m)) - 1) / SLOT;
+      sum_task<I, DT, VEC, G, UC>(a, decode_task(p, a.row_ptr, p.n_chunks + k), 0, stage);
+    }
 }
 
 // Combine split-row chunk partials in chunk order (deterministic).
@@ -357,52 +460,73 @@ __global__ __launch_bounds__(kTaskBlock) void sum_merge_kernel(
 }
 
 template <typename I, int DT, int VEC, int G>
-void launch_sum(const SumArgs<I, DT>& a, int64_t ftiles, hipStream_t s) {
+void launch_sum(const SumArgs<I, DT>& a, int tiles, hipStream_t s) {
   constexpr int U = (kWave / G) >= 16 ? 1 : (16 / (kWave / G) < 8 ? 16 / (kWave / G) : 8);
-  if constexpr (G <= 8) {
-    // ftiles == 1 here: G * VEC <= 32 covers F.
-    // One lane per edge (F = 1, or F = 4 as one 4-wide vector): 16-lane
-    // slots of 2 rows each, 8 rows per wave (the reference's F = 1 case,
-    // 131072 rows of 16 edges: 0.0254 ms with 32-lane slots of 2 rows,
-    // 0.0182 ms with these).  Wider rows: 32-lane slots of one row (two rows
-    // per wave measured 5% faster than four on 8-wide rows).
-    constexpr int SLOT = G == 1 ? 16 : 32;
+  const PlanView& p = a.plan;
+  // Rows of up to 8 lanes share a wave, and so do 16-lane rows of 16-bit
+  // values: they are shorter in time, so a row's fixed cost weighs more
+  // (12-edge rows of 100 bf16: 178 us a row per wave, 156 two, 116 four; 16
+  // lanes of fp32, 16-edge rows: 57, 58 and 61 us).
+  if constexpr (G <= 8 || (G == 16 && DT != TGX_DTYPE_F32)) {
+    // One lane per edge: 16-lane slots of 2 rows each, 8 rows per wave (the
+    // reference's F = 1 case, 131072 rows of 16 edges: 0.0254 ms with 32-lane
+    // slots of 2 rows, 0.0182 ms with these).  2 to 8 lanes: 32-lane slots of
+    // one row (two rows per wave measured 5% faster than four on 8-wide rows).
+    constexpr int SLOT = G == 1 || G == 16 ? 16 : 32;
     constexpr int P = G == 1 ? 2 : 1;
     constexpr int NS = kWave / SLOT;
-    const PlanView& p = a.plan;
+    constexpr int US = G < 8 ? G : 8;
     const int64_t waves = p.n_chunks + (p.n_wave + NS * P - 1) / (NS * P) +
                           (p.n_empty + kEmptyPerWave - 1) / kEmptyPerWave;
-    sum_pairs_kernel<I, DT, VEC, G, U, SLOT, P>
+    sum_pairs_kernel<I, DT, VEC, G, U, SLOT, P, US>
         <<<static_cast<unsigned>(ceil_div(waves, kWavesPerBlock)), kTaskBlock, 0, s>>>(a);
   } else {
-    const int64_t waves = plan_waves(a.plan);
-    dim3 grid(static_cast<unsigned>(ceil_div(waves, kWavesPerBlock)),
-              static_cast<unsigned>(ftiles));
+    const dim3 grid(static_cast<unsigned>(ceil_div(plan_waves(p), kWavesPerBlock)),
+                    static_cast<unsigned>(tiles));
     sum_rows_kernel<I, DT, VEC, G, U><<<grid, kTaskBlock, 0, s>>>(a);
   }
+}
+
+// Values per lane: 16 bytes, or what a narrower row has.
+inline int sum_vec(int64_t F, int dtype) {
+  if (F < 4) return 1;
+  return dtype == TGX_DTYPE_F32 || F < 8 ? 4 : 8;
+}
+
+// Feature tiles of 64 lanes (the widest) that cover a row.
+int sum_tiles(int64_t F, int dtype) {
+  return static_cast<int>(ceil_div(F, int64_t{kWave} * sum_vec(F, dtype)));
 }
 
 template <typename I, int DT>
 int sum_dispatch(const SumArgs<I, DT>& a, hipStream_t s) {
   const int64_t F = a.F;
-  if (F % 4 == 0) {
-    const int64_t lanes = F / 4;
-    if (lanes <= 1) launch_sum<I, DT, 4, 1>(a, 1, s);
-    else if (lanes <= 2) launch_sum<I, DT, 4, 2>(a, 1, s);
-    else if (lanes <= 4) launch_sum<I, DT, 4, 4>(a, 1, s);
-    else if (lanes <= 8) launch_sum<I, DT, 4, 8>(a, 1, s);
-    else if (lanes <= 16) launch_sum<I, DT, 4, 16>(a, 1, s);
-    else if (lanes <= 32) launch_sum<I, DT, 4, 32>(a, 1, s);
-    else launch_sum<I, DT, 4, 64>(a, ceil_div(lanes, 64), s);
-  } else {
-    if (F <= 1) launch_sum<I, DT, 1, 1>(a, 1, s);
-    else if (F <= 2) launch_sum<I, DT, 1, 2>(a, 1, s);
-    else if (F <= 4) launch_sum<I, DT, 1, 4>(a, 1, s);
-    else if (F <= 8) launch_sum<I, DT, 1, 8>(a, 1, s);
-    else if (F <= 16) launch_sum<I, DT, 1, 16>(a, 1, s);
-    else if (F <= 32) launch_sum<I, DT, 1, 32>(a, 1, s);
-    else launch_sum<I, DT, 1, 64>(a, ceil_div(F, 64), s);
-  }
+  const int vec = sum_vec(F, DT);
+  const int tiles = sum_tiles(F, DT);
+  int lanes = 1;
+  while (lanes < kWave && lanes < ceil_div(F, vec)) lanes *= 2;
+  const auto with_vec = [&](auto vc) {
+    constexpr int VEC = decltype(vc)::value;
+    switch (lanes) {
+      case 1: launch_sum<I, DT, VEC, 1>(a, tiles, s); break;
+      case 2: launch_sum<I, DT, VEC, 2>(a, tiles, s); break;
+      case 4: launch_sum<I, DT, VEC, 4>(a, tiles, s); break;
+      default:
+        // (Rows of fewer than 8 values have at most 4 lanes.)
+        if constexpr (VEC == (DT == TGX_DTYPE_F32 ? 4 : 8)) {
+          if (lanes == 8) launch_sum<I, DT, VEC, 8>(a, tiles, s);
+          else if (lanes == 16) launch_sum<I, DT, VEC, 16>(a, tiles, s);
+          else if (lanes == 32) launch_sum<I, DT, VEC, 32>(a, tiles, s);
+          else launch_sum<I, DT, VEC, 64>(a, tiles, s);
+        }
+    }
+  };
+  if (vec == 1)
+    with_vec(std::integral_constant<int, 1>{});
+  else if (vec == 4)
+    with_vec(std::integral_constant<int, 4>{});
+  else if constexpr (DT != TGX_DTYPE_F32)
+    with_vec(std::integral_constant<int, 8>{});
   TGX_LAUNCHED("sum_rows_kernel");
   if (a.plan.n_split > 0 && a.out) {
     sum_merge_kernel<DT><<<ceil_div(a.plan.n_split, kWavesPerBlock), kTaskBlock, 0, s>>>(
@@ -410,6 +534,27 @@ int sum_dispatch(const SumArgs<I, DT>& a, hipStream_t s) {
     TGX_LAUNCHED("sum_merge_kernel");
   }
   return TGX_OK;
+}
+
+// w_t[e'] = w[perm[e']]: the weights in transposed order, for launches that
+// read them once per feature tile.
+__global__ __launch_bounds__(kTaskBlock) void permute_weights_kernel(
+    const float* __restrict__ w, const int32_t* __restrict__ perm, int64_t n,
+    float* __restrict__ w_t) {
+  const int64_t e = static_cast<int64_t>(blockIdx.x) * kTaskBlock + threadIdx.x;
+  if (e < n) w_t[e] = w[perm[e]];
+}
+
+// dw[perm[e']] = the feature tiles' sums for edge e', in tile order.
+__global__ __launch_bounds__(kTaskBlock) void tile_dw_kernel(const float* __restrict__ part,
+                                                             int tiles, int64_t n,
+                                                             const int32_t* __restrict__ perm,
+                                                             float* __restrict__ dw) {
+  const int64_t e = static_cast<int64_t>(blockIdx.x) * kTaskBlock + threadIdx.x;
+  if (e >= n) return;
+  float s = 0.f;
+  for (int t = 0; t < tiles; ++t) s += part[t * n + e];
+  dw[perm[e]] = s;
 }
 
 // dw for feature widths that span several tiles: one wave per edge group of
@@ -497,18 +642,46 @@ extern "C" int tgx_csr_sum_fwd(const void* row_ptr, const void* col, int idx_bit
     typedef typename Elem<DT>::S S;
     SumArgs<I, DT> a{static_cast<const I*>(row_ptr), static_cast<const I*>(col),
                      plan_view(*plan), static_cast<const S*>(x), w, nullptr,
-                     static_cast<S*>(out), partial, nullptr, nullptr, F};
+                     static_cast<S*>(out), partial, nullptr, nullptr, nullptr, F, 0};
     return sum_dispatch(a, s);
   };
   return with_types(dtype, idx_bits, run);
 }
 
-extern "C" int tgx_csr_sum_bwd(const int32_t* row_ptr_t, const int32_t* col_t,
-                               const int32_t* perm, const tgx_row_plan* plan_t,
-                               const void* x, const float* w, const void* dout, void* dx,
-                               float* dw, int64_t n_dst, int64_t n_src, int64_t F, int dtype,
-                               float* partial, void* stream) {
-  TGX_REQUIRE(F > 0 && n_dst >= 0 && n_src >= 0, "bad sizes");
+// Workspace of a dw over several feature tiles: the tiles' dw and the weights
+// in transposed order.  Past kSumWorkspaceMax dw runs as a pass of its own.
+constexpr size_t kSumWorkspaceMax = size_t{2} << 30;
+
+struct SumBwdLayout {
+  int tiles;
+  size_t part_off, w_off, bytes;
+};
+
+static SumBwdLayout sum_bwd_layout(int64_t n_edges, int64_t F, int dtype) {
+  SumBwdLayout L{sum_tiles(F, dtype), 0, 0, 0};
+  if (L.tiles > 1) {
+    Carve c{nullptr, 0};
+    L.part_off = reinterpret_cast<size_t>(c.take<float>(L.tiles * n_edges));
+    L.w_off = reinterpret_cast<size_t>(c.take<float>(n_edges));
+    L.bytes = align_up(c.used) <= kSumWorkspaceMax ? align_up(c.used) : 0;
+  }
+  return L;
+}
+
+extern "C" int tgx_csr_sum_bwd_workspace(int64_t n_edges, int64_t F, int dtype, size_t* bytes) {
+  TGX_REQUIRE(bytes, "null bytes");
+  TGX_REQUIRE(F > 0 && n_edges >= 0, "bad sizes");
+  *bytes = sum_bwd_layout(n_edges, F, dtype).bytes;
+  return TGX_OK;
+}
+
+extern "C" int tgx_csr_sum_bwd_ws(const int32_t* row_ptr_t, const int32_t* col_t,
+                                  const int32_t* perm, const tgx_row_plan* plan_t,
+                                  const void* x, const float* w, const void* dout, void* dx,
+                                  float* dw, int64_t n_dst, int64_t n_src, int64_t n_edges,
+                                  int64_t F, int dtype, float* partial, void* ws,
+                                  size_t ws_bytes, void* stream) {
+  TGX_REQUIRE(F > 0 && n_dst >= 0 && n_src >= 0 && n_edges >= 0, "bad sizes");
   if (dtype != TGX_DTYPE_F32 && dtype != TGX_DTYPE_BF16 && dtype != TGX_DTYPE_F16) {
     set_error("sum supports fp32, bf16 and fp16 features (dtype code %d)", dtype);
     return TGX_UNSUPPORTED;
@@ -521,22 +694,45 @@ extern "C" int tgx_csr_sum_bwd(const int32_t* row_ptr_t, const int32_t* col_t,
   TGX_REQUIRE(!dw || x, "dw needs x");
   TGX_REQUIRE(plan_t->n_chunks == 0 || partial || !dx, "split rows need a partial buffer");
   hipStream_t s = as_stream(stream);
-  const bool single_tile = (F % 4 == 0) ? (F / 4 <= 64) : (F <= 64);
+  const SumBwdLayout L = sum_bwd_layout(n_edges, F, dtype);
+  const bool tiled = L.bytes > 0 && ws && ws_bytes >= L.bytes && n_edges > 0;
+  float* const part = tiled ? reinterpret_cast<float*>(static_cast<char*>(ws) + L.part_off)
+                            : nullptr;
   TGX_PROFILE("csr_sum_bwd", s);
   auto run = [&](auto dt, auto) -> int {
     constexpr int DT = decltype(dt)::value;
     typedef typename Elem<DT>::S S;
     const S* xs = static_cast<const S*>(x);
     const S* gs = static_cast<const S*>(dout);
-    if (dx) {
+    const bool with_dw = dw && (L.tiles == 1 || tiled);   // dw from the sum's own pass
+    if (dx || with_dw) {
       SumArgs<int32_t, DT> a{row_ptr_t, col_t, plan_view(*plan_t), gs, w, perm,
-                             static_cast<S*>(dx), partial,
-                             (dw && single_tile) ? xs : nullptr,
-                             (dw && single_tile) ? dw : nullptr, F};
+                             static_cast<S*>(dx), partial, nullptr, nullptr, nullptr, F, 0};
+      if (tiled) {
+        if (w) {
+          float* w_t = reinterpret_cast<float*>(static_cast<char*>(ws) + L.w_off);
+          permute_weights_kernel<<<ceil_div(n_edges, kTaskBlock), kTaskBlock, 0, s>>>(
+              w, perm, n_edges, w_t);
+          TGX_LAUNCHED("permute_weights_kernel");
+          a.w = w_t;
+        }
+        a.wperm = nullptr;
+      }
+      if (with_dw) {
+        a.self_x = xs;
+        a.dw = tiled ? part : dw;
+        a.dwperm = tiled ? nullptr : perm;
+        a.dw_tile = tiled ? n_edges : 0;
+      }
       const int r = sum_dispatch(a, s);
       if (r != TGX_OK) return r;
+      if (tiled && with_dw) {
+        tile_dw_kernel<<<ceil_div(n_edges, kTaskBlock), kTaskBlock, 0, s>>>(part, L.tiles, n_edges,
+                                                                            perm, dw);
+        TGX_LAUNCHED("tile_dw_kernel");
+      }
     }
-    if (dw && (!dx || !single_tile)) {
+    if (dw && !with_dw) {
       sum_dw_wide_kernel<DT><<<ceil_div(n_src, kWavesPerBlock), kTaskBlock, 0, s>>>(
           row_ptr_t, col_t, perm, xs, gs, dw, n_src, F);
       TGX_LAUNCHED("sum_dw_wide_kernel");
@@ -544,6 +740,15 @@ extern "C" int tgx_csr_sum_bwd(const int32_t* row_ptr_t, const int32_t* col_t,
     return TGX_OK;
   };
   return with_types(dtype, 32, run);
+}
+
+extern "C" int tgx_csr_sum_bwd(const int32_t* row_ptr_t, const int32_t* col_t,
+                               const int32_t* perm, const tgx_row_plan* plan_t,
+                               const void* x, const float* w, const void* dout, void* dx,
+                               float* dw, int64_t n_dst, int64_t n_src, int64_t F, int dtype,
+                               float* partial, void* stream) {
+  return tgx_csr_sum_bwd_ws(row_ptr_t, col_t, perm, plan_t, x, w, dout, dx, dw, n_dst, n_src, 0,
+                            F, dtype, partial, nullptr, 0, stream);
 }
 
 extern "C" int tgx_csr_edge_dot(const void* row_ptr, const void* col, int idx_bits,
@@ -576,7 +781,7 @@ extern "C" int tgx_csr_edge_dot(const void* row_ptr, const void* col, int idx_bi
     // writes dw[e] = <dout[i], x[col[e]]> in edge order and no sums.
     SumArgs<I, DT> a{static_cast<const I*>(row_ptr), static_cast<const I*>(col),
                      plan_view(*plan), static_cast<const S*>(x), nullptr, nullptr, nullptr,
-                     nullptr, static_cast<const S*>(dout), dw, F};
+                     nullptr, static_cast<const S*>(dout), dw, nullptr, F, 0};
     return sum_dispatch(a, s);
   };
   return with_types(dtype, idx_bits, run);

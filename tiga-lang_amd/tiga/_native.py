@@ -84,6 +84,9 @@ _SIGNATURES: dict[str, list] = {
                         c_i64, c_int, c_vp, c_vp],
     "tgx_csr_sum_bwd": [c_vp, c_vp, c_vp, P(RowPlan), c_vp, c_vp, c_vp, c_vp, c_vp,
                         c_i64, c_i64, c_i64, c_int, c_vp, c_vp],
+    "tgx_csr_sum_bwd_workspace": [c_i64, c_i64, c_int, P(c_size)],
+    "tgx_csr_sum_bwd_ws": [c_vp, c_vp, c_vp, P(RowPlan), c_vp, c_vp, c_vp, c_vp, c_vp, c_i64,
+                           c_i64, c_i64, c_i64, c_int, c_vp, c_vp, c_size, c_vp],
     "tgx_csr_edge_dot": [c_vp, c_vp, c_int, P(RowPlan), c_vp, c_vp, c_vp, c_i64, c_i64, c_i64,
                          c_int, c_vp],
     "tgx_gat_fwd": [c_vp, c_vp, c_int, P(RowPlan), c_vp, c_vp, c_vp, c_vp, c_f32, c_vp,

@@ -149,10 +149,19 @@ class CsrSumFunction(torch.autograd.Function):
         if n_src and ctx.F and (need_dx or (E and not dw_in_csr)):
             t = graph._transposed()
             partial = _partial(t.plan, ctx.F, xc.device) if need_dx else None
-            _native.call("tgx_csr_sum_bwd", t.row_ptr_t.data_ptr(), t.col_t.data_ptr(),
+            code = _native.dtype_code(xc)
+            ws, ws_size = None, 0
+            if dw is not None and not dw_in_csr:
+                ws_bytes = ctypes.c_size_t()
+                _native.call("tgx_csr_sum_bwd_workspace", E, ctx.F, code,
+                             ctypes.byref(ws_bytes))
+                ws_size = ws_bytes.value
+                if ws_size:
+                    ws = torch.empty(ws_size, dtype=torch.uint8, device=xc.device)
+            _native.call("tgx_csr_sum_bwd_ws", t.row_ptr_t.data_ptr(), t.col_t.data_ptr(),
                          t.perm.data_ptr(), t.plan.ref, xc.data_ptr(), _p(wc),
                          dout.data_ptr(), _p(dx), None if dw_in_csr else _p(dw), n_dst,
-                         n_src, ctx.F, _native.dtype_code(xc), _p(partial),
+                         n_src, E, ctx.F, code, _p(partial), _p(ws), ws_size,
                          _native.stream_of(xc))
         if dw_in_csr:
             row_ptr, col_idx = graph._kernel_csr()
