@@ -88,8 +88,12 @@ __device__ __forceinline__ Task decode_task(const PlanView& p, const I* row_ptr,
   return t;
 }
 
+// The wave's index in the launch, known to be the same for its 64 lanes: the
+// task's decode, its row list and row pointer reads and the edge loops' bounds
+// then run on the scalar unit.
 __device__ __forceinline__ int64_t global_wave() {
-  return static_cast<int64_t>(blockIdx.x) * kWavesPerBlock + threadIdx.x / kWave;
+  return static_cast<int64_t>(blockIdx.x) * kWavesPerBlock +
+         uniform(static_cast<int>(threadIdx.x / kWave));
 }
 
 }  // namespace tgx
