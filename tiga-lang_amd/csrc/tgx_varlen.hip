@@ -74,11 +74,22 @@ using vec4 = typename Vec<T>::v4;
 
 constexpr int VBM = 128;   // queries per workgroup (4 waves x 32)
 constexpr int VBN = 64;    // keys per iteration
-// LDS row stride (elements) of every staged tile: 288 B rows keep both the
-// 16 B row-fragment reads and the transposing 8 B reads free of bank
-// conflicts (measured: SQ_LDS_BANK_CONFLICT = 0).  D = 64 uses the first half
-// of each row.
+// LDS row stride (elements) of a staged tile: 288 B rows keep both the 16 B
+// row-fragment reads and the transposing 8 B reads free of bank conflicts
+// (measured: SQ_LDS_BANK_CONFLICT = 0).  The backward's narrower heads use the
+// first part of each row.
 constexpr int TPAD = 144;
+// The forward's, by head dim, and the workgroups per CU its registers are held
+// to: 160 and 96 B rows are as free of conflicts (eight rows fall on distinct
+// banks), and with 288 B ones the double-buffered K and V tiles left room for
+// two workgroups per CU at every D.  24 causal sequences of 500 to 2000
+// tokens: D = 64, 12 heads 125 -> 110 us, D = 32, 16 heads 118 -> 96 us.  (The
+// backward's tiles are single-buffered and not bound by LDS capacity: the same
+// rows there measured 273 -> 282 us.)
+template <int D>
+constexpr int FPAD = D == 128 ? 144 : D == 64 ? 80 : 48;
+template <int D>
+constexpr int kFwdWaves = D == 128 ? 2 : D == 64 ? 3 : 4;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 // gfx950 (MI355X) has 8 XCDs, each with its own L2; workgroup i of a launch
@@ -192,9 +203,8 @@ __device__ __forceinline__ void stage_load(Stage<T, D>& st, const T* xa, int64_t
   }
 }
 
-template <typename T, int D>
-__device__ __forceinline__ void stage_store(const Stage<T, D>& st, T (*ra)[TPAD],
-                                            T (*rb)[TPAD]) {
+template <typename T, int D, int PAD>
+__device__ __forceinline__ void stage_store(const Stage<T, D>& st, T (*ra)[PAD], T (*rb)[PAD]) {
   constexpr int CPR = D / 8;
 #pragma unroll
   for (int it = 0; it < Stage<T, D>::N; ++it) {
@@ -205,14 +215,14 @@ __device__ __forceinline__ void stage_store(const Stage<T, D>& st, T (*ra)[TPAD]
 }
 
 // A fragment of X^T (rows of X are the contraction index) from a row-major
-// LDS tile X[row][col] with row stride TPAD: lane (lr, g) receives
+// LDS tile X[row][col] with row stride PAD: lane (lr, g) receives
 // X[r0 + 4g + j][c0 + lr] for j < 4 and X[r0 + 16 + 4g + j - 4][c0 + lr] for
 // j >= 4, i.e. 8 rows of one column in the permuted order of the B operand.
-template <typename T>
-__device__ __forceinline__ vec8<T> tr_frag(T (*x)[TPAD], int r0, int c0, int lr, int g) {
+template <typename T, int PAD>
+__device__ __forceinline__ vec8<T> tr_frag(T (*x)[PAD], int r0, int c0, int lr, int g) {
   const T* p = &x[r0 + 4 * g + (lr >> 2)][c0 + 4 * (lr & 3)];
   const i16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(p));
-  const i16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(p + 16 * TPAD));
+  const i16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(p + 16 * PAD));
   // Assemble at dword granularity (elements 0-3 from a, 4-7 from b).
   const u32x2 aw = __builtin_bit_cast(u32x2, a);
   const u32x2 bw = __builtin_bit_cast(u32x2, b);
@@ -254,11 +264,11 @@ template <int D>
 constexpr int64_t kPartialFloats = static_cast<int64_t>(VBM) * (D + 2);
 
 template <typename T, int D, bool CAUSAL, bool PRUNE>
-__global__ __launch_bounds__(256, 2) void varlen_fwd_kernel(FwdArgs<T> a) {
+__global__ __launch_bounds__(256, kFwdWaves<D>) void varlen_fwd_kernel(FwdArgs<T> a) {
   constexpr int KC = D / 32;   // contraction steps of S over D
   constexpr int DT = D / 16;   // 16-row tiles of O^T
-  __shared__ T ks[2][VBN][TPAD];
-  __shared__ T vs[2][VBN][TPAD];
+  __shared__ T ks[2][VBN][FPAD<D>];
+  __shared__ T vs[2][VBN][FPAD<D>];
   __shared__ float wave_max[PRUNE ? 4 : 1];
   const int32_t* task = a.tasks + 4 * static_cast<int64_t>(blockIdx.x);
   const int blk = task[0];
