@@ -390,6 +390,52 @@ def test_gat_element_types_and_bipartite_parity(H, D, dtype, bipartite, a_typed)
     assert rel_err(f(a_d.grad), e_dad) <= a_tol
 
 
+# Tables of over 512 MB run the gathers one half of the heads after the other:
+# the last table that does not and the first that does (1 KB rows), and heads
+# that fill a lane group (nothing to halve).
+@pytest.mark.parametrize("n_src,H,D", [(524_288, 8, 32), (524_289, 8, 32), (524_289, 2, 128),
+                                       (524_289, 1, 256), (524_289, 3, 128)])
+@pytest.mark.parametrize("bipartite", [False, True])
+def test_gat_halved_head_groups(n_src, H, D, bipartite):
+    """Few edges over large tables, hub rows and hub sources split into
+    chunks, against float64 autograd (fp32 tolerance)."""
+    print(f"gat halves N={n_src} H={H} D={D} bipartite={bipartite}", flush=True)
+    n_dst = 600_000 if bipartite else n_src
+    g = torch.Generator(device=DEV).manual_seed(H)
+    rows = torch.randint(0, n_dst, (60_000,), device=DEV, generator=g)
+    rows[:2500] = 7
+    cols = torch.randint(0, n_src, (60_000,), device=DEV, generator=g)
+    cols[3000:5000] = n_src - 1
+    rows, order = torch.sort(rows)
+    cols = cols[order]
+    row_ptr = torch.zeros(n_dst + 1, dtype=torch.int64, device=DEV)
+    row_ptr[1:] = torch.cumsum(torch.bincount(rows, minlength=n_dst), 0)
+    graph = tg.Graph.from_csr(row_ptr, cols, num_src=n_src)
+    h = torch.randn(n_src, H, D, device=DEV, generator=g).requires_grad_(True)
+    hd = (torch.randn(n_dst, H, D, device=DEV, generator=g).requires_grad_(True)
+          if bipartite else h)
+    a_s, a_d = (0.1 * torch.randn(H, D, device=DEV, generator=g) for _ in range(2))
+    leaves = [h, hd, a_s.requires_grad_(True), a_d.requires_grad_(True)]
+    dout = torch.randn(n_dst, H, D, device=DEV, generator=g)
+    out = GAT(a_s, a_d, 0.2)(graph=graph, src={"h": h}, dst={"h": hd})
+    grads = torch.autograd.grad(out, leaves if bipartite else [h, a_s, a_d], dout)
+    h64, hd64, as64, ad64 = (t.detach().double().requires_grad_(True) for t in leaves)
+    if not bipartite:
+        hd64 = h64
+    z = (h64[cols] * as64).sum(-1) + (hd64[rows] * ad64).sum(-1)
+    score = F.leaky_relu(z, 0.2)
+    top = torch.full((n_dst, H), -float("inf"), dtype=torch.float64, device=DEV).scatter_reduce(
+        0, rows[:, None].expand_as(score), score.detach(), "amax")
+    p = torch.exp(score - top[rows])
+    alpha = p / torch.zeros_like(top).index_add(0, rows, p)[rows]
+    want = torch.zeros(n_dst, H, D, dtype=torch.float64, device=DEV).index_add(
+        0, rows, alpha[..., None] * h64[cols])
+    want_grads = torch.autograd.grad(want, [h64, hd64, as64, ad64] if bipartite
+                                     else [h64, as64, ad64], dout.double())
+    for got, exp in zip([out.detach(), *grads], [want.detach(), *want_grads]):
+        assert float((got.double() - exp).abs().max() / exp.abs().max()) <= RTOL32
+
+
 def test_gat_large_scores_and_determinism():
     # Scores of order 1e3 (the reference's overflow case) must stay finite.
     N, H, D = 600, 8, 32

@@ -55,6 +55,8 @@
 // becomes a node pass over h for da_src and da_dst.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "tgx_device.h"
 #include "tgx_host.h"
 #include "tgx_profile.h"
@@ -339,6 +341,7 @@ struct GatSrcArgs {
   const float* sdz_dst;  // MODE 2: [N, H] from B1
   int64_t ld;       // values between consecutive nodes' rows of hs, dout, dh
   int64_t nsld;     // floats between consecutive nodes' rows of ns
+  int64_t sld;      // floats between consecutive nodes' rows of sdz_src, sdz_dst
 };
 
 // One wave per task of the transposed-CSR plan (source rows).  MODE 0: dz
@@ -364,12 +367,12 @@ __global__ __launch_bounds__(kTaskBlock, MODE ? 7 : 1) void gat_bwd_src_kernel(
       const int64_t j = uniform(a.plan.rows[t.empty0 + k]);
       if (g == 0) {
         if constexpr (MODE == 2)
-          V::store(a.dhs + j * a.ld + 4 * c, a.sdz_dst[j * H + hd] * ld4(a.a_dst + 4 * c));
+          V::store(a.dhs + j * a.ld + 4 * c, a.sdz_dst[j * a.sld + hd] * ld4(a.a_dst + 4 * c));
         else if (a.dh_acc)
           st4(a.dh_acc + j * a.ld + 4 * c, f32x4{0.f, 0.f, 0.f, 0.f});
         else
           V::store(a.dhs + j * a.ld + 4 * c, f32x4{0.f, 0.f, 0.f, 0.f});
-        if (head_lead) a.sdz_src[j * H + hd] = 0.f;
+        if (head_lead) a.sdz_src[j * a.sld + hd] = 0.f;
       }
     }
     return;
@@ -429,12 +432,12 @@ __global__ __launch_bounds__(kTaskBlock, MODE ? 7 : 1) void gat_bwd_src_kernel(
     if (head_lead) p[HD + hd] = sdz;
   } else {
     // (Folded modes run with dh_acc == null: dh is final here.)
-    if constexpr (MODE == 2) contrib = contrib + a.sdz_dst[j * H + hd] * ld4(a.a_dst + 4 * c);
+    if constexpr (MODE == 2) contrib = contrib + a.sdz_dst[j * a.sld + hd] * ld4(a.a_dst + 4 * c);
     if (a.dh_acc)
       st4(a.dh_acc + j * a.ld + 4 * c, contrib);
     else
       V::store(a.dhs + j * a.ld + 4 * c, contrib);
-    if (head_lead) a.sdz_src[j * H + hd] = sdz;
+    if (head_lead) a.sdz_src[j * a.sld + hd] = sdz;
   }
 }
 
@@ -443,7 +446,8 @@ template <int DT, int G, int HL, bool FOLD>
 __global__ __launch_bounds__(kTaskBlock) void gat_bwd_src_merge_kernel(
     PlanView plan, const float* __restrict__ partial, float* __restrict__ dh_acc,
     typename Vals<DT, 4>::T* __restrict__ dhs, float* __restrict__ sdz_src,
-    const float* __restrict__ a_dst, const float* __restrict__ sdz_dst, int64_t ld) {
+    const float* __restrict__ a_dst, const float* __restrict__ sdz_dst, int64_t ld,
+    int64_t sld) {
   using V = Vals<DT, 4>;
   constexpr int HD = 4 * G;
   constexpr int H = G / HL;
@@ -475,12 +479,12 @@ __global__ __launch_bounds__(kTaskBlock) void gat_bwd_src_merge_kernel(
         z += pz[u];
       }
   }
-  if constexpr (FOLD) s = s + sdz_dst[row * H + hd] * ld4(a_dst + 4 * c);
+  if constexpr (FOLD) s = s + sdz_dst[row * sld + hd] * ld4(a_dst + 4 * c);
   if (dh_acc)
     st4(dh_acc + row * ld + 4 * c, s);
   else
     V::store(dhs + row * ld + 4 * c, s);
-  if (c % HL == 0) sdz_src[row * H + hd] = z;
+  if (c % HL == 0) sdz_src[row * sld + hd] = z;
 }
 
 template <int DT, typename I>
@@ -820,6 +824,20 @@ struct GatBwdIo {
   int64_t col_off;   // the head group's first column (h0 * D) within a row
 };
 
+// fp32 rows of 1 KB (64 lanes) of a table over twice the Infinity Cache (256
+// MB): the gather passes run one half of the heads after the other.  Each pass
+// then gathers 512 bytes a row from half the bytes, twice as much of which the
+// cache holds, and its lines come at the L2s' rate (7 TB/s) where whole rows
+// wait for HBM (6.1 TB/s).  1M nodes, 17M edges, 8 heads of 32: forward 3.19 ->
+// 2.76 ms, source pass 3.56 -> 3.37 ms, edges read twice.  Quarters: 3.33 and
+// 4.22 ms; tables of 512 MB and less gain nothing (random rows alone: 500,000
+// of 1 KB 7.1 TB/s whole, 6.9 halved).
+template <int DT, int G, int HL>
+constexpr bool can_halve = DT == TGX_DTYPE_F32 && G == 64 && HL <= G / 2;
+bool halve_heads(int64_t table_rows, int row_floats) {
+  return table_rows * row_floats * 4 > (int64_t{512} << 20);
+}
+
 // Node-pass grid: one wave per EPW nodes, at most what stays resident.
 template <class Kernel>
 int64_t node_blocks(Kernel k, int64_t n, int epw) {
@@ -833,9 +851,6 @@ int gat_bwd_launch(const I* row_ptr, const tgx_row_plan& plan, const int32_t* ro
                    const GatBwdLayout& L, hipStream_t s) {
   using T = typename Vals<DT, 4>::T;
   constexpr int EPW = kWave / G;
-  // The source pass holds dout rows plus node state per edge: 4 in flight
-  // per wave measured best (2: +4%, 3: +2%, 6: +5%, 8: +6% time).
-  constexpr int U = EPW >= 4 ? 1 : 4 / EPW;
   constexpr int HD = 4 * G;
   const bool homogeneous = io.dhs == io.dhd;
   const bool folded = io.pos != nullptr;
@@ -871,24 +886,51 @@ int gat_bwd_launch(const I* row_ptr, const tgx_row_plan& plan, const int32_t* ro
     TGX_LAUNCHED("gat_delta_kernel");
   }
 
-  const GatSrcArgs<DT> sa{row_ptr_t, col_t, perm, pt, hs, io.a_src, io.slope, io.ns,
-                          static_cast<const T*>(io.dout), dh_acc, static_cast<T*>(io.dhs),
-                          src_part, dz, sdz_src, io.a_dst, sdz_dst, io.ld, io.nsld};
-  if (plan_waves(pt) > 0) {
-    TGX_PROFILE("gat_bwd_src_kernel", s);
-    const auto k = src_mode == 0 ? gat_bwd_src_kernel<DT, G, HL, U, 0>
-                   : src_mode == 1 ? gat_bwd_src_kernel<DT, G, HL, U, 1>
-                                   : gat_bwd_src_kernel<DT, G, HL, U, 2>;
-    k<<<ceil_div(plan_waves(pt), kWavesPerBlock), kTaskBlock, 0, s>>>(sa);
-    TGX_LAUNCHED("gat_bwd_src_kernel");
+  // The source pass over heads [h, h + 4 GG / D) of the group.
+  auto src_pass = [&](auto gg, int h) -> int {
+    constexpr int GG = decltype(gg)::value;
+    // dout rows plus node state per edge: 4 in flight per wave measured best
+    // (2: +4%, 3: +2%, 6: +5%, 8: +6% time).
+    constexpr int US = kWave / GG >= 4 ? 1 : 4 * GG / kWave;
+    const int64_t off = static_cast<int64_t>(h) * 4 * HL;
+    float* acc = dh_acc ? dh_acc + off : nullptr;
+    T* dhs = static_cast<T*>(io.dhs) + off;
+    const float* sdst = sdz_dst ? sdz_dst + h : nullptr;
+    const GatSrcArgs<DT> sa{row_ptr_t, col_t, perm, pt, hs + off, io.a_src + off, io.slope,
+                            io.ns + 4 * h, static_cast<const T*>(io.dout) + off, acc, dhs,
+                            src_part, dz, sdz_src + h, io.a_dst + off, sdst, io.ld, io.nsld,
+                            G / HL};
+    if (plan_waves(pt) > 0) {
+      TGX_PROFILE("gat_bwd_src_kernel", s);
+      const auto k = src_mode == 0 ? gat_bwd_src_kernel<DT, GG, HL, US, 0>
+                     : src_mode == 1 ? gat_bwd_src_kernel<DT, GG, HL, US, 1>
+                                     : gat_bwd_src_kernel<DT, GG, HL, US, 2>;
+      k<<<ceil_div(plan_waves(pt), kWavesPerBlock), kTaskBlock, 0, s>>>(sa);
+      TGX_LAUNCHED("gat_bwd_src_kernel");
+    }
+    if (pt.n_split > 0) {
+      TGX_PROFILE("gat_bwd_src_merge_kernel", s);
+      const auto k = src_mode == 2 ? gat_bwd_src_merge_kernel<DT, GG, HL, true>
+                                   : gat_bwd_src_merge_kernel<DT, GG, HL, false>;
+      k<<<ceil_div(pt.n_split, kWavesPerBlock), kTaskBlock, 0, s>>>(
+          pt, src_part, acc, dhs, sdz_src + h, io.a_dst + off, sdst, io.ld, G / HL);
+      TGX_LAUNCHED("gat_bwd_src_merge_kernel");
+    }
+    return TGX_OK;
+  };
+  bool halves = false;
+  if constexpr (can_halve<DT, G, HL>) {
+    if (folded && halve_heads(io.n_dst, HD)) {
+      halves = true;
+      for (int h : {0, G / HL / 2}) {
+        const int st = src_pass(std::integral_constant<int, G / 2>{}, h);
+        if (st != TGX_OK) return st;
+      }
+    }
   }
-  if (pt.n_split > 0) {
-    TGX_PROFILE("gat_bwd_src_merge_kernel", s);
-    const auto k = src_mode == 2 ? gat_bwd_src_merge_kernel<DT, G, HL, true>
-                                 : gat_bwd_src_merge_kernel<DT, G, HL, false>;
-    k<<<ceil_div(pt.n_split, kWavesPerBlock), kTaskBlock, 0, s>>>(
-        pt, src_part, dh_acc, static_cast<T*>(io.dhs), sdz_src, io.a_dst, sdz_dst, io.ld);
-    TGX_LAUNCHED("gat_bwd_src_merge_kernel");
+  if (!halves) {
+    const int st = src_pass(std::integral_constant<int, G>{}, 0);
+    if (st != TGX_OK) return st;
   }
 
   int64_t src_blocks = 0, dst_blocks = 0;
@@ -961,12 +1003,13 @@ int gat_bwd_launch(const I* row_ptr, const tgx_row_plan& plan, const int32_t* ro
 template <int DT>
 int gat_fwd_dtype(const void* row_ptr, const void* col, int idx_bits, const tgx_row_plan* plan,
                   const void* hs, const void* hd, const float* a_src, const float* a_dst,
-                  float slope, void* out, float* ns, int H, int D, float* partial,
-                  float* pos, hipStream_t s) {
+                  float slope, void* out, float* ns, int64_t n_src, int H, int D,
+                  float* partial, float* pos, hipStream_t s) {
   using T = typename Vals<DT, 4>::T;
   const int64_t ld = static_cast<int64_t>(H) * D, nsld = 4 * static_cast<int64_t>(H);
   for (int h0 = 0; h0 < H;) {
-    const int hg = gat_group_heads(H, D, h0);
+    int hg = gat_group_heads(H, D, h0);
+    if (DT == TGX_DTYPE_F32 && hg >= 2 && hg * D == 256 && halve_heads(n_src, hg * D)) hg /= 2;
     const GatShape shp = gat_shape(hg, D);
     const int64_t off = static_cast<int64_t>(h0) * D;
     const T* hs_g = hs ? static_cast<const T*>(hs) + off : nullptr;
@@ -1085,13 +1128,13 @@ extern "C" int tgx_gat_fwd(const void* row_ptr, const void* col, int idx_bits,
   switch (dtype) {
     case TGX_DTYPE_F32:
       return gat_fwd_dtype<TGX_DTYPE_F32>(row_ptr, col, idx_bits, plan, h_src, h_dst, a_src,
-                                          a_dst, slope, out, ns, H, D, partial, pos, s);
+                                          a_dst, slope, out, ns, n_src, H, D, partial, pos, s);
     case TGX_DTYPE_BF16:
       return gat_fwd_dtype<TGX_DTYPE_BF16>(row_ptr, col, idx_bits, plan, h_src, h_dst, a_src,
-                                           a_dst, slope, out, ns, H, D, partial, pos, s);
+                                           a_dst, slope, out, ns, n_src, H, D, partial, pos, s);
     default:
       return gat_fwd_dtype<TGX_DTYPE_F16>(row_ptr, col, idx_bits, plan, h_src, h_dst, a_src,
-                                          a_dst, slope, out, ns, H, D, partial, pos, s);
+                                          a_dst, slope, out, ns, n_src, H, D, partial, pos, s);
   }
 }
 
