@@ -604,6 +604,40 @@ int tgx_edge_mlp_scores(const void* col_dev, const int32_t* dst_index_dev, int i
                         int64_t n_edges, const tgx_edge_mlp* mlp, float* scores_dev,
                         void* stream);
 
+/* Two-layer networks over destination fields with the first layer's destination
+ * columns applied once per row instead of once per edge: scores as tgx_edge_mlp_scores gives them, up to fp32 rounding, and
+ * the attention backward as tgx_edge_mlp_attention_backward's, except that
+ * destination fields' gradients come back per row.
+ *   tgx_edge_mlp_projected_state: floats of the state buffer (16-byte
+ *     aligned) the scores fill and the backward reads; TGX_UNSUPPORTED where
+ *     the kernels do not cover the chain (two layers, up to 16 hidden units,
+ *     functions up to TGX_ACT_MISH but TGX_ACT_HARDTANH, no LayerNorm, source
+ *     fields of up to 8 floats in all, destination fields of 1 to 16, edge
+ *     fields of up to 7, at most two of a role): the caller then uses
+ *     the entry points above, as it may for any chain.
+ *   tgx_edge_mlp_projected_scores: the layers as they are, w1 [hidden, inputs],
+ *     b1 [hidden] or NULL, w2 [hidden], b2 [1] or NULL (mlp->weights_dev is not
+ *     read).
+ *   tgx_edge_mlp_projected_backward: dseg[s] is [n_edges, width] for source
+ *     and edge segments (the folded segment's rows with alpha dout added) and
+ *     [n_dst, width], final, for destination segments; row_ptr is the CSR's;
+ *     out, dout, value 16-byte aligned; dweights in the padded layout. */
+int tgx_edge_mlp_projected_state(int64_t n_dst, const tgx_edge_mlp* mlp, int64_t* floats);
+int tgx_edge_mlp_projected_scores(const void* col_dev, const int32_t* dst_index_dev,
+                                  int idx_bits, int64_t n_edges, int64_t n_dst,
+                                  const tgx_edge_mlp* mlp, const float* w1_dev,
+                                  const float* b1_dev, const float* w2_dev,
+                                  const float* b2_dev, float* state_dev, float* scores_dev,
+                                  void* stream);
+int tgx_edge_mlp_projected_workspace(int64_t n_edges, int64_t n_dst, const tgx_edge_mlp* mlp,
+                                     size_t* bytes);
+int tgx_edge_mlp_projected_backward(
+    const void* row_ptr_dev, const void* col_dev, const int32_t* dst_index_dev, int idx_bits,
+    int64_t n_edges, int64_t n_dst, const tgx_edge_mlp* mlp, float* state_dev,
+    const float* lse_dev, const float* out_dev, const float* dout_dev, const float* value_dev,
+    int32_t value_width, int fold_segment, float* dweights_dev, float* const* dseg_dev,
+    void* workspace_dev, size_t workspace_bytes, void* stream);
+
 /* Edge-network messages summed per destination row (the reference's
  * edge-NN tile, python/tiga/compiler/edge_nn_tile.py:1-30, dispatched by
  * interop/torch/message_passing.py:2134-2300: tg.sum() over

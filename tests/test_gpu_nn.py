@@ -342,3 +342,104 @@ def test_graph_without_edges():
     assert torch.count_nonzero(x.grad) == 0
     for p in attn.parameters():
         assert p.grad is not None and torch.count_nonzero(p.grad) == 0
+
+
+class ProjectedScore(tg.MessagePassing):
+    """Scores over up to five fields in a given order; the value is the source
+    field "x" (whose score gradient is folded in) or a constant "v"."""
+
+    reducer = tg.online_softmax()
+
+    def __init__(self, net, order, value):
+        super().__init__()
+        self.net = tg.nn.trace(net)
+        self.order, self.value = order, value
+
+    def edge(self, src, dst, edge):
+        at = {"x": lambda: src.x, "s": lambda: src.s, "y": lambda: dst.y, "d": lambda: dst.d,
+              "e": lambda: edge.e, "f": lambda: edge.f}
+        return self.reducer(self.net(*[at[k]() for k in self.order]),
+                            src.x if self.value == "x" else src.v)
+
+
+# (rows, mean degree, hub, widths of the fields in the order that they are
+# given in, hidden, activation, index type, value).  Widths and hidden sizes at
+# the limits and inside; rows of degree 1, rows over many waves of 64 edges and
+# workgroups of 256, edge counts no multiple of either.
+PROJECTED = [
+    (300, 9, 700, {"e": 3, "x": 8, "y": 8}, 16, nn.LeakyReLU(0.2), torch.int64, "x"),
+    (301, 1.2, 0, {"y": 16, "x": 8, "e": 7}, 16, nn.LeakyReLU(0.1), torch.int32, "x"),
+    (3, 40, 3000, {"x": 4, "y": 1}, 1, nn.ReLU(), torch.int32, "x"),
+    (257, 30, 0, {"y": 5, "x": 3, "d": 4, "e": 2}, 17, nn.ReLU(), torch.int64, "x"),
+    (129, 64, 0, {"s": 2, "y": 3, "x": 6}, 8, nn.ELU(0.7), torch.int32, "x"),
+    (200, 17, 257, {"y": 2, "e": 3, "d": 1, "f": 2}, 13, nn.GELU(), torch.int32, "v"),
+    (64, 1, 1, {"x": 1, "y": 13}, 15, nn.Tanh(), torch.int64, "x"),
+    (90, 12, 64, {"x": 8, "y": 7, "e": 1}, 16, nn.SiLU(), torch.int64, "x"),
+]
+
+
+@pytest.mark.parametrize("rows,degree,hub,fields,hidden,act,index,value", PROJECTED)
+@pytest.mark.parametrize("bias", [True, False])
+def test_projected_first_layer(monkeypatch, rows, degree, hub, fields, hidden, act, index, value,
+                               bias):
+    """The kernels that apply the first layer's destination columns once per
+    row, and the per-edge kernels on the same inputs, against 64 bits."""
+    from tiga import _ops
+
+    print("projected", rows, degree, hub, fields, hidden, act, index, value, bias, flush=True)
+    torch.manual_seed(rows)
+    n_src = rows + 11
+    rp, col = random_graph(rows, n_src, degree, rows, hub=hub, empty=0.05)
+    graph = tg.Graph.from_csr(rp.to(index), col.to(index), num_src=n_src)
+    E = graph.num_edges
+    count = {"x": n_src, "s": n_src, "v": n_src, "y": rows, "d": rows, "e": E, "f": E}
+    net = nn.Sequential(nn.Linear(sum(fields.values()), hidden, bias=bias), act,
+                        nn.Linear(hidden, 1, bias=bias)).to(DEV)
+    data = {k: torch.randn(count[k], w) for k, w in fields.items()}
+    if value == "v":
+        data["v"] = torch.randn(n_src, 5)
+    width = data[value].shape[1]
+    dout = torch.randn(rows, width)
+
+    # 64 bits, on the CPU.
+    net64 = nn.Sequential(*[m for m in net]).double().cpu()
+    wide = {k: t.double().requires_grad_(k != "v") for k, t in data.items()}
+    c, r = col.cpu().long(), torch.repeat_interleave(torch.arange(rows), rp.cpu().diff())
+    at = {"x": c, "s": c, "y": r, "d": r, "e": slice(None), "f": slice(None)}
+    score = net64(torch.cat([wide[k][at[k]] for k in fields], 1)).squeeze(1)
+    top = torch.full((rows,), -torch.inf, dtype=torch.float64).scatter_reduce(
+        0, r, score.detach(), "amax")
+    ex = (score - top[r]).exp()
+    alpha = ex / torch.zeros(rows, dtype=torch.float64).index_add(0, r, ex)[r]
+    expect = torch.zeros(rows, width, dtype=torch.float64).index_add(
+        0, r, alpha[:, None] * wide[value][c])
+    params64 = list(net64.parameters())
+    expect_grads = torch.autograd.grad(expect, [wide[k] for k in fields] + params64,
+                                       dout.double())
+    net = net64.float().to(DEV)
+
+    used = []
+    find = _ops._projected_state
+    for projected in (True, False):
+        monkeypatch.setattr(_ops, "_projected_state",
+                            (lambda *a: used.append(find(*a)) or used[-1]) if projected
+                            else (lambda *a: None))
+        args = {k: t.to(DEV).requires_grad_(k != "v") for k, t in data.items()}
+        kernel = ProjectedScore(net, tuple(fields), value)
+        out = kernel(graph=graph, **{
+            role: {k: args[k] for k in names if k in args}
+            for role, names in (("src", "xsv"), ("dst", "yd"), ("edge", "ef"))})
+        grads = torch.autograd.grad(out, [args[k] for k in fields] + list(net.parameters()),
+                                    dout.to(DEV))
+        assert rel_err(f64(out), expect.detach()) <= RTOL
+        for k, g, e in zip(fields, grads, expect_grads):
+            assert rel_err(f64(g), e) <= RTOL, (projected, k)
+        n = len(fields)
+        for p, g, e in zip(params64, grads[n:], expect_grads[n:]):
+            # The last bias's gradient is 0: in the scale of its weight's.
+            scale = max(float(e.abs().max()),
+                        float(expect_grads[-2 if bias else -1].abs().max()) if p.numel() == 1
+                        else 0.0, 1e-30)
+            assert float((g.double().cpu() - e).abs().max()) <= 3e-5 * scale, (projected, p.shape)
+    # The rule's edges: hidden 17 and fewer edges than rows stay per edge.
+    assert used and all((u is not None) == (E >= rows and hidden <= 16) for u in used)

@@ -130,6 +130,13 @@ _SIGNATURES: dict[str, list] = {
     "tgx_edge_mlp_hidden": [c_vp, c_vp, c_int, c_i64, P(EdgeMlp), c_vp, ctypes.c_int32, c_vp],
     "tgx_edge_mlp_backward_seeded": [c_vp, c_vp, c_int, c_i64, P(EdgeMlp), c_vp,
                                      ctypes.c_int32, c_vp, P(c_vp), c_vp, c_size, c_vp],
+    "tgx_edge_mlp_projected_state": [c_i64, P(EdgeMlp), P(c_i64)],
+    "tgx_edge_mlp_projected_scores": [c_vp, c_vp, c_int, c_i64, c_i64, P(EdgeMlp), c_vp, c_vp,
+                                      c_vp, c_vp, c_vp, c_vp, c_vp],
+    "tgx_edge_mlp_projected_workspace": [c_i64, c_i64, P(EdgeMlp), P(c_size)],
+    "tgx_edge_mlp_projected_backward": [c_vp, c_vp, c_vp, c_int, c_i64, c_i64, P(EdgeMlp),
+                                        c_vp, c_vp, c_vp, c_vp, c_vp, ctypes.c_int32, c_int, c_vp,
+                                        P(c_vp), c_vp, c_size, c_vp],
     "tgx_segment_softmax_fwd": [c_vp, c_int, c_i64, c_vp, c_vp, c_vp, c_vp],
     "tgx_segment_softmax_bwd": [c_vp, c_int, c_i64, c_vp, c_vp, c_vp, c_vp],
     "tgx_segment_softmax_gather_fwd": [c_vp, c_vp, c_int, c_i64, c_vp, c_int, c_f32, c_vp,

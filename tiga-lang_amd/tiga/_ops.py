@@ -531,7 +531,7 @@ def _mlp_struct(chain, roles, segs, weights_buf, width):
         # The last layer of an edge-network sum is applied by the caller;
         # the kernels see it as a one-output layer they do not evaluate.
         m.out_width[l] = layer.linear.out_features if l + 1 < len(chain) else 1
-    m.weights_dev = weights_buf.data_ptr()
+    m.weights_dev = _p(weights_buf)
     m.n_segments = len(segs)
     for s, (role, seg) in enumerate(zip(roles, segs)):
         m.seg_role[s] = _ROLE[role]
@@ -631,14 +631,15 @@ def _layer_grads(chain, dweights, W, present, needs, first, layers):
     return grads
 
 
-def _segment_grads(graph, roles, dsegs, shapes, needs, first):
-    """Per-edge input-segment gradients reduced onto their fields' rows."""
+def _segment_grads(graph, roles, dsegs, shapes, needs, first, dst_rows=False):
+    """Per-edge input-segment gradients reduced onto their fields' rows
+    (dst_rows: destination fields' come reduced)."""
     grads = []
     for s, (role, d, shape) in enumerate(zip(roles, dsegs, shapes)):
         if not needs[first + s]:
             grads.append(None)
             continue
-        if role == "edge":
+        if role == "edge" or (role == "dst" and dst_rows):
             g = d
         elif role == "src":
             g = _reduce_rows_transposed(graph, d)
@@ -708,6 +709,25 @@ class SegmentSoftmaxFunction(torch.autograd.Function):
         return dscore, None
 
 
+def _projected_state(graph: Graph, mlp, E: int, device) -> torch.Tensor | None:
+    """The state buffer of the kernels that apply the first layer's
+    destination columns once per row (tgx_edge_mlp_projected_*), or None where
+    the chain is not theirs.  They work per row too, so a graph
+    of fewer edges than rows stays with the per-edge network (training step of
+    19-16-1, value 8: 29 edges a row, 131k rows 447 us against 630; one edge a
+    row 290 against 341, both the host's launches)."""
+    n_dst = graph.schema.num_dst
+    if mlp.n_layers != 2 or E < n_dst:
+        return None
+    floats = ctypes.c_int64()
+    try:
+        _native.call("tgx_edge_mlp_projected_state", n_dst, ctypes.byref(mlp),
+                     ctypes.byref(floats))
+    except NotImplementedError:
+        return None
+    return torch.empty(floats.value, dtype=torch.float32, device=device)
+
+
 class NnAttentionFunction(torch.autograd.Function):
     """out[i] = sum_e softmax_i(net(fields_e)) value[col[e]], fp32, with the
     logsumexp-recompute backward.  The forward keeps per destination row only
@@ -732,31 +752,11 @@ class NnAttentionFunction(torch.autograd.Function):
         E, n_dst = col_idx.numel(), graph.schema.num_dst
         W = _padded_width(chain, sum(s.shape[1] for s in segs))
         dev = col_idx.device
-        buf = torch.zeros(len(chain), _block_floats(chain, W), dtype=torch.float32, device=dev)
-        _fill_weights(buf, chain, params, W, len(chain))
-        mlp = _mlp_struct(chain, roles, segs, buf, W)
+        mlp = _mlp_struct(chain, roles, segs, None, W)
         stream = _native.stream_of(col_idx)
-        # The scores live only for this forward; value rows of at most 8
-        # floats are summed in the softmax pass itself (no per-edge weight
-        # is written), wider ones by the CSR sum over the weights.
-        scores = torch.empty(E, dtype=torch.float32, device=dev)
-        _native.call("tgx_edge_mlp_scores", col_idx.data_ptr(), graph._dst_index32().data_ptr(),
-                     _native.idx_bits(row_ptr), E, ctypes.byref(mlp), scores.data_ptr(), stream)
-        lse = torch.empty(max(n_dst, 1), dtype=torch.float32, device=dev)
-        out = _fused_softmax_sum(graph, scores, TGX_ROLE_EDGE, 1.0, value, lse)
-        if out is not None:
-            vc, F = _aligned(value), 1
-            for d in value.shape[1:]:
-                F *= d
-        else:
-            alpha = torch.empty_like(scores)
-            _native.call("tgx_segment_softmax_fwd", row_ptr.data_ptr(),
-                         _native.idx_bits(row_ptr), n_dst, scores.data_ptr(), alpha.data_ptr(),
-                         lse.data_ptr(), stream)
-            out, vc, _, F = _csr_sum_launch(value, alpha, graph)
-            del alpha
-        del scores
-        ctx.graph, ctx.chain, ctx.roles, ctx.n_seg, ctx.W, ctx.F = graph, chain, roles, n_seg, W, F
+        F = 1
+        for d in value.shape[1:]:
+            F *= d
         # A value that is also a source field of the score (the reference's
         # GAT example: value src.x, score over src.x): its two gradients meet
         # per edge in the backward kernel, so one transposed reduction
@@ -764,9 +764,49 @@ class NnAttentionFunction(torch.autograd.Function):
         ctx.fold = next((i for i in range(n_seg)
                          if roles[i] == "src" and tensors[i] is value
                          and segs[i].shape[1] == F), -1)
+        # The projected kernels write no per-edge weight: they take the value
+        # gradient folded, or none.
+        state = (_projected_state(graph, mlp, E, dev)
+                 if ctx.fold >= 0 or not ctx.needs_input_grad[4] else None)
+        buf = None
+        if state is None:
+            buf = torch.zeros(len(chain), _block_floats(chain, W), dtype=torch.float32,
+                              device=dev)
+            _fill_weights(buf, chain, params, W, len(chain))
+            mlp.weights_dev = buf.data_ptr()
+        # The scores live only for this forward; value rows of at most 8
+        # floats are summed in the softmax pass itself (no per-edge weight
+        # is written), wider ones by the CSR sum over the weights.
+        scores = torch.empty(E, dtype=torch.float32, device=dev)
+        if state is not None:
+            layers = [None if x is None else x.to(dev, torch.float32).contiguous()
+                      for l in range(2)
+                      for x in _folded(chain[l], params[_PER_LAYER * l],
+                                       params[_PER_LAYER * l + 1])]
+            _native.call("tgx_edge_mlp_projected_scores", col_idx.data_ptr(),
+                         graph._dst_index32().data_ptr(), _native.idx_bits(row_ptr), E,
+                         n_dst, ctypes.byref(mlp), *map(_p, layers), state.data_ptr(), scores.data_ptr(), stream)
+        else:
+            _native.call("tgx_edge_mlp_scores", col_idx.data_ptr(),
+                         graph._dst_index32().data_ptr(), _native.idx_bits(row_ptr), E,
+                         ctypes.byref(mlp), scores.data_ptr(), stream)
+        lse = torch.empty(max(n_dst, 1), dtype=torch.float32, device=dev)
+        out = _fused_softmax_sum(graph, scores, TGX_ROLE_EDGE, 1.0, value, lse)
+        if out is not None:
+            vc = _aligned(value)
+        else:
+            alpha = torch.empty_like(scores)
+            _native.call("tgx_segment_softmax_fwd", row_ptr.data_ptr(),
+                         _native.idx_bits(row_ptr), n_dst, scores.data_ptr(), alpha.data_ptr(),
+                         lse.data_ptr(), stream)
+            out, vc, _, _ = _csr_sum_launch(value, alpha, graph)
+            del alpha
+        del scores
+        ctx.graph, ctx.chain, ctx.roles, ctx.n_seg, ctx.W, ctx.F = graph, chain, roles, n_seg, W, F
         ctx.shapes = [t.shape for t in tensors[:n_seg]]
         ctx.present = [t is not None for t in params]
-        ctx.save_for_backward(buf, lse, out, vc, *segs)
+        ctx.projected = state is not None
+        ctx.save_for_backward(state if ctx.projected else buf, lse, out, vc, *segs)
         return out
 
     @staticmethod
@@ -781,15 +821,33 @@ class NnAttentionFunction(torch.autograd.Function):
         fold = ctx.fold if ctx.needs_input_grad[4] else -1
         alpha = (torch.empty(max(E, 1), dtype=torch.float32, device=dev)
                  if ctx.needs_input_grad[4] and fold < 0 else None)
-        dsegs = [torch.empty(E, s.shape[1], dtype=torch.float32, device=dev) for s in segs]
-        mlp = _mlp_struct(chain, roles, segs, buf, W)
+        projected = ctx.projected   # (then alpha is None)
+        dsegs = [torch.empty(n_dst if projected and role == "dst" else E, s.shape[1],
+                             dtype=torch.float32, device=dev) for role, s in zip(roles, segs)]
+        mlp = _mlp_struct(chain, roles, segs, None if projected else buf, W)
         ws_bytes = ctypes.c_size_t()
-        _native.call("tgx_edge_mlp_backward_workspace", E, ctypes.byref(mlp),
-                     ctypes.byref(ws_bytes))
+        if projected:
+            _native.call("tgx_edge_mlp_projected_workspace", E, n_dst, ctypes.byref(mlp),
+                         ctypes.byref(ws_bytes))
+        else:
+            _native.call("tgx_edge_mlp_backward_workspace", E, ctypes.byref(mlp),
+                         ctypes.byref(ws_bytes))
         ws = torch.empty(max(ws_bytes.value, 4), dtype=torch.uint8, device=dev)
-        dweights = torch.empty(L, buf.shape[1], dtype=torch.float32, device=dev)
+        dweights = torch.empty(L, _block_floats(chain, W), dtype=torch.float32, device=dev)
         ptrs = (ctypes.c_void_p * 4)(*[d.data_ptr() for d in dsegs], *([None] * (4 - len(dsegs))))
         stream = _native.stream_of(col_idx)
+        if projected:
+            _native.call("tgx_edge_mlp_projected_backward", row_ptr.data_ptr(),
+                         col_idx.data_ptr(), graph._dst_index32().data_ptr(),
+                         _native.idx_bits(row_ptr), E, n_dst, ctypes.byref(mlp),
+                         buf.data_ptr(), lse.data_ptr(), out.data_ptr(), g.data_ptr(),
+                         vc.data_ptr(), F, fold, dweights.data_ptr(), ptrs, ws.data_ptr(),
+                         ws_bytes.value, stream)
+            grads = _segment_grads(graph, roles, dsegs, ctx.shapes, ctx.needs_input_grad, 5,
+                                   dst_rows=True)
+            grads += _layer_grads(chain, dweights, W, ctx.present, ctx.needs_input_grad,
+                                  5 + ctx.n_seg, L)
+            return (None, None, None, None, None, *grads)
         _native.call("tgx_edge_mlp_attention_backward", col_idx.data_ptr(),
                      graph._dst_index32().data_ptr(), _native.idx_bits(row_ptr), E,
                      ctypes.byref(mlp), lse.data_ptr(), out.data_ptr(), g.data_ptr(),
