@@ -25,10 +25,13 @@
 // gradient alpha dout[i] added), as tgx_edge_mlp_attention_backward writes.
 // Every sum has a fixed order.
 //
-// 131,072 nodes, 3.9M edges, 19-16-1, leaky ReLU, value 8 folded (MI355X; the
-// edge-MLP kernels in parentheses): scores 64 us, backward 213, rows and weights
-// 35; forward and backward of the
-// layer, with the softmax and the transposed sum, 630 -> 447
+// 131,072 nodes, 3.9M edges, 19-16-1, leaky ReLU, value 8 folded (MI355X):
+// scores 63 us, backward 214, rows and weights 35; forward and backward of the
+// layer, with the softmax and the transposed sum, 447 us (630 on the edge-MLP
+// kernels).  The edge pass is bound by the gathered lines (about 73 us of it) and
+// by the exposed latency of its chain of loads, weights and LDS sums at four
+// waves a SIMD: with a third fewer instructions (arguments read from the
+// argument segment instead of spilled) it took 214 us against 224.
 #include <hip/hip_runtime.h>
 
 #include "tgx_nn_common.h"

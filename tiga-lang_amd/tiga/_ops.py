@@ -717,7 +717,7 @@ def _projected_state(graph: Graph, mlp, E: int, device) -> torch.Tensor | None:
     19-16-1, value 8: 29 edges a row, 131k rows 447 us against 630; one edge a
     row 290 against 341, both the host's launches)."""
     n_dst = graph.schema.num_dst
-    if mlp.n_layers != 2 or E < n_dst:
+    if mlp.n_layers != 2 or E < max(n_dst, 1):
         return None
     floats = ctypes.c_int64()
     try:
