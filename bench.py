@@ -527,8 +527,9 @@ def run_c2(args):
     bytes_per = gat_kernel_bytes(N, E, H, D)
     step_bytes = sum(bytes_per.values())
     dominant = max((k for k in per_kernel if k in bytes_per), key=lambda k: per_kernel[k][1])
-    n_launch, total_ms = per_kernel[dominant]
-    avg_ms = total_ms / n_launch
+    # Per step, as the bytes are: the gather passes of a table this size are two
+    # launches, one per half of the heads.
+    avg_ms = per_kernel[dominant][1] / args.steps
     achieved = bytes_per[dominant] / (avg_ms * 1e-3) / 1e9
     ms_per_step = elapsed * 1e3 / args.steps
     result = {
@@ -554,8 +555,9 @@ def run_c2(args):
                      "traffic": measured_traffic("c2", dominant)[0],
                      "traffic_source": measured_traffic("c2", dominant)[1], "avg_ms": avg_ms,
                      "algorithmic_bytes": bytes_per[dominant]},
-        "kernels": {k: {"launches": n, "avg_ms": ms / n,
-                        "gbs": (bytes_per[k] / (ms / n * 1e-3) / 1e9) if k in bytes_per else None}
+        "kernels": {k: {"launches": n, "avg_ms": ms / args.steps,
+                        "gbs": (bytes_per[k] / (ms / args.steps * 1e-3) / 1e9)
+                               if k in bytes_per else None}
                     for k, (n, ms) in sorted(per_kernel.items())},
     }
     result["profiled_ms_per_step"] = profiled * 1e3 / args.steps
@@ -1000,11 +1002,15 @@ def run_nn(args):
     # score pass reads col, dst, the 19 input floats (displacement 3, x_src 8,
     # x_dst 8) and writes the score; the backward reads the same plus dscore
     # and writes the 19 input-gradient floats (the weight gradients are summed
-    # on chip).
+    # on chip).  The kernels that apply x_dst's columns once per row read and
+    # write it per row instead (score pass: its 16 products' row written and
+    # read; backward: the row sums of dz, the gradient rows come after it).
     inputs = 4 * (3 + 8 + 8)
     bytes_per = {
         "edge_mlp_fwd_kernel": E * (4 + 4 + inputs + 4),
         "edge_mlp_bwd_kernel": E * (4 + 4 + inputs + 4 + inputs),
+        "projected_scores_kernel": E * (4 + 4 + 12 + 32 + 4) + N * 64,
+        "projected_bwd_kernel": E * (4 + 4 + 2 * (12 + 32)) + N * (64 + 64 + 4 + 4 + 64),
         "csr_sum_fwd": E * (4 + 4 + 32) + N * (4 + 32),
     }
     per = totals
@@ -1027,7 +1033,8 @@ def run_nn(args):
                      "traffic_source": measured_traffic("nn", dominant)[1],
                      "algorithmic_bytes": bytes_per[dominant],
                      "note": "the edge MLP kernels are issue- and latency-bound fp32 work "
-                             "(weights in scalar registers), far from the HBM roof"},
+                             "(weights in scalar registers) on 32-byte gathered rows, far "
+                             "from the HBM roof"},
         "kernels": {k: {"launches": n, "avg_ms": t / n} for k, (n, t) in sorted(per.items())},
     }
     result["profiled_ms_per_step"] = profiled * 1e3 / args.steps
