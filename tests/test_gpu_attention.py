@@ -14,6 +14,7 @@ import pytest
 import torch
 
 import tiga as tg
+from tiga import _native
 from oracle import ref
 
 pytestmark = pytest.mark.gpu
@@ -312,3 +313,27 @@ def test_split_key_ranges_match_whole_tiles(n, H, D, causal, dtype):
         assert float((got - expect).abs().max() / expect.abs().max()) <= tol
     for a, b in zip(results[0], results[1]):
         assert float((a - b).abs().max() / b.abs().max()) <= tol
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_split_forward_launches_the_graphs_one_list(monkeypatch, D):
+    """The first forward of a graph builds one split list (a call for its
+    sizes, one for its entries), whatever the head dim, and launches that list:
+    chunks do not depend on how many narrow-head workgroups a CU holds."""
+    print(f"split list D={D}", flush=True)
+    calls = []
+    call = _native.call
+    monkeypatch.setattr(_native, "call",
+                        lambda name, *args: (calls.append((name, args)), call(name, *args))[1])
+    g = torch.Generator(device=DEV).manual_seed(D)
+    q, k, v = (torch.randn(4096, 4, D, device=DEV, generator=g).to(torch.float16)
+               for _ in range(3))
+    graph = tg.Graph.triangular(4096, device=DEV)
+    with torch.no_grad():
+        DotAttention()(graph=graph, src={"key": k, "value": v}, dst={"query": q},
+                       scale=D ** -0.5)
+    names = [name for name, _ in calls]
+    assert names.count("tgx_attn_fwd_split_tasks") == 2
+    launch = dict(calls)["tgx_attn_fwd_split"]
+    tasks, n, merge, n_merge, chunk, max_chunks = graph._attn_fwd_split(4)
+    assert launch[2:8] == (tasks.data_ptr(), n, merge.data_ptr(), n_merge, chunk, max_chunks)

@@ -1100,18 +1100,17 @@ template <typename T, int D>
 int launch_fwd(const AttnShape& s, FwdArgs<T> a, int64_t n_tasks, bool prune,
                hipStream_t stream) {
   const unsigned grid = static_cast<unsigned>(n_tasks);
+  // Split lists are cut to two workgroups' load per CU: with a third one's room
+  // some CUs take three of them and others one (4096 causal tokens, 16 heads of
+  // 64: 62.9 us a call against 59.3 with the room taken up by unused LDS).
+  const unsigned lds =
+      a.chunk_tiles > 0 ? 4 * VBN * (TPAD - FPAD<D>) * static_cast<unsigned>(sizeof(T)) : 0;
   TGX_PROFILE("varlen_fwd_kernel", stream);
-  if (s.causal) {
-    if (prune)
-      varlen_fwd_kernel<T, D, true, true><<<grid, 256, 0, stream>>>(a);
-    else
-      varlen_fwd_kernel<T, D, true, false><<<grid, 256, 0, stream>>>(a);
-  } else {
-    if (prune)
-      varlen_fwd_kernel<T, D, false, true><<<grid, 256, 0, stream>>>(a);
-    else
-      varlen_fwd_kernel<T, D, false, false><<<grid, 256, 0, stream>>>(a);
-  }
+  const auto k = s.causal ? (prune ? varlen_fwd_kernel<T, D, true, true>
+                                   : varlen_fwd_kernel<T, D, true, false>)
+                          : (prune ? varlen_fwd_kernel<T, D, false, true>
+                                   : varlen_fwd_kernel<T, D, false, false>);
+  k<<<grid, 256, lds, stream>>>(a);
   TGX_LAUNCHED("varlen_fwd_kernel");
   return TGX_OK;
 }

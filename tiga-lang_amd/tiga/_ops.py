@@ -338,8 +338,6 @@ STORED_DS_MAX_BYTES = 8 << 30
 # Keys per dK/dV workgroup of the attention backward (the key task lists of
 # tgx_attn_tasks, kind 1, are built with this block).
 ATTN_KEY_TILE = 64
-# Resident forward workgroups per CU by head dim (registers and LDS).
-ATTN_FWD_PER_CU = {32: 4, 64: 3}
 
 
 class BlockAttentionFunction(torch.autograd.Function):
@@ -358,12 +356,6 @@ class BlockAttentionFunction(torch.autograd.Function):
         out = torch.empty((n_q, H, D), dtype=q.dtype, device=q.device)
         lse = torch.empty((n_q, H), dtype=torch.float32, device=q.device)
         split = None if prune > 0 else graph._attn_fwd_split(H)
-        if split is not None and D < 128:
-            # Narrower heads keep more workgroups resident: finer chunks.  (Not
-            # where two per CU run whole tiles: the merge would cost more than
-            # the third gains, 108 -> 111 us for 4096 dense tokens, 16 heads of
-            # 64; 72 -> 69 us where the causal tiles are split anyway.)
-            split = graph._attn_fwd_split(H, ATTN_FWD_PER_CU[D])
         if split is not None:
             # Too few, too uneven query tiles: the longest key ranges run in
             # chunks, merged afterwards (tgx_attn_fwd_split).

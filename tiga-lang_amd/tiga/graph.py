@@ -805,21 +805,17 @@ class Graph:
             self._native_cache[key] = got
         return got
 
-    def _attn_fwd_split(self, heads: int, per_cu: int = 2):
+    def _attn_fwd_split(self, heads: int):
         """The forward's split-key-range task lists for a `heads`-head launch
-        (tgx_attn_fwd_split_tasks with `per_cu` resident workgroups per CU):
+        (tgx_attn_fwd_split_tasks with two resident workgroups per CU):
         (tasks, n_tasks, merge, n_merge, chunk_tiles, max_chunks) on the
-        device, or None when no tile is worth splitting.  (None kept under
-        ("attn-split", heads) turns splitting off for the graph.)"""
-        if self._native_cache.get(("attn-split", heads), True) is None:
-            return None
-        key = ("attn-split", heads, per_cu)
+        device, or None when no tile is worth splitting."""
+        key = ("attn-split", heads)
         if key not in self._native_cache:
             import numpy as np
 
             cu_q, cu_k, causal = self._attn_blocks()
-            cus = torch.cuda.get_device_properties(self.device).multi_processor_count
-            slots = per_cu * cus
+            slots = 2 * torch.cuda.get_device_properties(self.device).multi_processor_count
             n, n_merge = ctypes.c_int64(), ctypes.c_int64()
             chunk, max_chunks = ctypes.c_int32(), ctypes.c_int32()
             args = (cu_q.ctypes.data, cu_k.ctypes.data, cu_q.size - 1, heads, int(causal),
