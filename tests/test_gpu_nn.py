@@ -443,3 +443,31 @@ def test_projected_first_layer(monkeypatch, rows, degree, hub, fields, hidden, a
             assert float((g.double().cpu() - e).abs().max()) <= 3e-5 * scale, (projected, p.shape)
     # The rule's edges: hidden 17 and fewer edges than rows stay per edge.
     assert used and all((u is not None) == (E >= rows and hidden <= 16) for u in used)
+
+
+@pytest.mark.parametrize("dst_width", [1, 8, 13])
+@pytest.mark.parametrize("bad", [torch.inf, torch.nan])
+def test_rows_without_edges_may_hold_anything(dst_width, bad):
+    """A destination row without edges takes no part in the layer: Inf or NaN
+    in its fields reaches neither the weights' gradients nor its own, which
+    are the bits that finite values there give."""
+    print(f"projected, isolated rows of {bad}, width {dst_width}", flush=True)
+    torch.manual_seed(dst_width)
+    rows, n_src = 70, 90
+    rp, col = random_graph(rows, n_src, 9, 5, hub=100, empty=0.3)
+    graph = tg.Graph.from_csr(rp, col, num_src=n_src)
+    empty = rp.to(DEV).diff() == 0
+    assert graph.num_edges >= rows and empty.any()
+    net = nn.Sequential(nn.Linear(8 + dst_width, 16), nn.LeakyReLU(0.2), nn.Linear(16, 1)).to(DEV)
+    kernel = ProjectedScore(net, ("x", "y"), "x")
+    x = torch.randn(n_src, 8, device=DEV).requires_grad_(True)
+    y = torch.randn(rows, dst_width, device=DEV)
+    dout = torch.randn(rows, 8, device=DEV)
+    got = []
+    for value in (0.0, bad):
+        yv = torch.where(empty[:, None], torch.full_like(y, value), y).requires_grad_(True)
+        out = kernel(graph=graph, src={"x": x}, dst={"y": yv}, edge={})
+        got.append([out, *torch.autograd.grad(out, [x, yv, *net.parameters()], dout)])
+    for a, b in zip(*got):
+        assert torch.isfinite(a).all() and torch.equal(a, b)
+    assert torch.count_nonzero(got[1][2][empty]) == 0

@@ -595,17 +595,18 @@ __global__ __launch_bounds__(256) void projected_rows_kernel(const I* __restrict
        first += step) {
     const int64_t row = first + q;
     const bool valid = row < n_rows;
+    const int64_t r0 = valid ? row_ptr[row] : 0, r1 = valid ? row_ptr[row + 1] : 0;
+    // A row without edges has no part in the layer: its fields are not read
+    // (they may be Inf or NaN, a mean over no neighbours) and its gradient is 0.
+    const bool any = r1 > r0;
     float dz = 0.f, u = 0.f;
-    if (valid) {
-      const int64_t r0 = row_ptr[row], r1 = row_ptr[row + 1];
-      if (r1 > r0) {
-        const int64_t w0 = r0 / kWave, w1 = (r1 - 1) / kWave;
-        if (w0 == w1) {
-          dz = dzt[row * HP + hh];
-        } else {
-          dz = part[(w0 * 2 + 1) * HP + hh];
-          for (int64_t w = w0 + 1; w <= w1; ++w) dz += part[w * 2 * HP + hh];
-        }
+    if (any) {
+      const int64_t w0 = r0 / kWave, w1 = (r1 - 1) / kWave;
+      if (w0 == w1) {
+        dz = dzt[row * HP + hh];
+      } else {
+        dz = part[(w0 * 2 + 1) * HP + hh];
+        for (int64_t w = w0 + 1; w <= w1; ++w) dz += part[w * 2 * HP + hh];
       }
       if (x) u = x[row * stride];
     }
@@ -613,7 +614,7 @@ __global__ __launch_bounds__(256) void projected_rows_kernel(const I* __restrict
 #pragma unroll
     for (int h = 0; h < HP; ++h) g = fmaf(wt[h], __shfl(dz, 16 * q + h, kWave), g);
     acc = __builtin_amdgcn_mfma_f32_16x16x4f32(dz, u, acc, 0, 0, 0);
-    if (valid && x) grad[row * width] = g;
+    if (valid && x) grad[row * width] = any ? g : 0.f;
   }
 #pragma unroll
   for (int r = 0; r < 4; ++r) red[wave][(4 * q + r) * kU + hh] = acc[r];
