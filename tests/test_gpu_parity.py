@@ -278,6 +278,42 @@ def test_sum_width_and_tile_edges(n_dst, n_src, F_, dtype):
     assert torch.equal(dx, dx_only) and torch.equal(dw, dw_only)
 
 
+# Widths that are no multiple of a lane's values (4 fp32, 8 16-bit), of narrow
+# rows, whole-wave rows and several tiles.
+@pytest.mark.parametrize("F_", [5, 30, 100, 300, 514, 1030])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_edge_weight_gradients_of_infinite_values(F_, dtype):
+    """An infinite output gradient or feature makes its edges' dw Inf of the
+    product's sign, wherever in the row it lies: dw's dot products take each
+    value once.  Both passes that write dw: beside dx and on its own."""
+    print(f"infinite values F={F_} {dtype}", flush=True)
+    rp, col = skewed_csr(F_, 400, 300, mean_deg=5, hubs=(1300, 129))
+    graph = tg.Graph.from_csr(to_dev(rp, torch.int64), to_dev(col, torch.int64), num_src=300)
+    rows, cols = graph.destination_index(), to_dev(col, torch.int64)
+    g = torch.Generator(device=DEV).manual_seed(F_)
+    from tiga._ops import CsrSumFunction
+
+    for in_dout in (True, False):
+        x = 0.5 + torch.rand(300, F_, device=DEV, generator=g).to(dtype)
+        dout = 0.5 + torch.rand(400, F_, device=DEV, generator=g).to(dtype)
+        w = torch.rand(col.size, device=DEV, generator=g)
+        t = dout if in_dout else x
+        place = torch.arange(t.shape[0], device=DEV)
+        t[place[::3], place[::3] % F_] = torch.inf
+        t[place[1::3], F_ - 1 - place[1::3] % min(F_, 8)] = -torch.inf
+        want = (x[cols].double() * dout[rows].double()).sum(1)
+        for x_grad in (True, False):
+            xg, wg = x.clone().requires_grad_(x_grad), w.clone().requires_grad_(True)
+            out = CsrSumFunction.apply(xg, wg, graph)
+            (dw,) = torch.autograd.grad(out, (wg,), dout)
+            assert not torch.isnan(dw).any()
+            assert torch.equal(torch.isposinf(dw), torch.isposinf(want))
+            assert torch.equal(torch.isneginf(dw), torch.isneginf(want))
+            finite = torch.isfinite(want)
+            assert float((dw.double() - want)[finite].abs().max()) <= \
+                RTOL32 * float(want[finite].abs().max())
+
+
 # ---- GAT additive ----------------------------------------------------------
 
 class GAT(tg.MessagePassing):

@@ -192,8 +192,32 @@ __device__ __forceinline__ float dot(const float (&a)[VEC], const float (&b)[VEC
   return s;
 }
 
+// A second look at the dw of edges e, e + step, ... < e1 of a row, where some
+// came out NaN: an infinite repeated value times the 0 of load_self is NaN where
+// the sum may be Inf.  Those are formed again from the two rows' columns
+// [first, end), each once.  (The gather loops only note that there is one, and
+// launches without dw have kernels of their own: fp16 F = 11, 2.7M edges fwd +
+// bwd 232 us before this, 230 so; with a select per gathered value, or all of it
+// in one kernel, 244.)
+template <typename I, int DT>
+__device__ __forceinline__ void redo_nan_dw(const SumArgs<I, DT>& a, int64_t row, int64_t e,
+                                            int64_t e1, int step, int64_t dw_off, int64_t first,
+                                            int64_t end) {
+  const typename Elem<DT>::S* const self = a.self_x + row * a.F;
+#pragma unroll 1
+  for (; e < e1; e += step) {
+    float* const to = a.dw + dw_off + (a.dwperm ? static_cast<int64_t>(a.dwperm[e]) : e);
+    if (*to == *to) continue;
+    const typename Elem<DT>::S* const x = a.x + (a.col ? static_cast<int64_t>(a.col[e]) : e) * a.F;
+    float s = 0.f;
+#pragma unroll 1
+    for (int64_t k = first; k < end; ++k) s += Elem<DT>::load1(x + k) * Elem<DT>::load1(self + k);
+    *to = s;
+  }
+}
+
 // One whole-wave task (a row, a split-row chunk or a group of empty rows).
-template <typename I, int DT, int VEC, int G, int U>
+template <typename I, int DT, int VEC, int G, int U, bool DW>
 __device__ __forceinline__ void sum_task(const SumArgs<I, DT>& a, const Task& t, int tile,
                                          float* dw_stage) {
   typedef Vec<VEC, DT> V;
@@ -216,11 +240,11 @@ __device__ __forceinline__ void sum_task(const SumArgs<I, DT>& a, const Task& t,
   }
 
   float self[VEC] = {};
-  const bool want_dw = a.self_x != nullptr;
-  if (want_dw && lc.active)
+  if (DW && lc.active)
     load_self<VEC, DT>(a.self_x + static_cast<int64_t>(t.row) * F, lc, self);
 
   float acc[VEC] = {};
+  bool nan = false;   // this lane wrote a dw that is NaN
   for (int64_t base = t.e0; base < t.e1; base += kWave) {
     const int n = static_cast<int>(t.e1 - base < kWave ? t.e1 - base : kWave);
     int my_col = 0;
@@ -255,13 +279,13 @@ __device__ __forceinline__ void sum_task(const SumArgs<I, DT>& a, const Task& t,
 #pragma unroll
           for (int q = 0; q < VEC; ++q) acc[q] += wt[u] * f[q];
         }
-        if (want_dw) {
+        if constexpr (DW) {
           const float d = group_sum<G>(dot(f, self));
           if (c == 0 && slot[u] < n) dw_stage[slot[u]] = d;
         }
       }
     }
-    if (want_dw) {
+    if constexpr (DW) {
       // A window's dw values wait in LDS and leave with one store per lane
       // after the window, not one store per edge group inside the gather loop
       // (whose following gathers would share its in-order completion count).
@@ -271,9 +295,18 @@ __device__ __forceinline__ void sum_task(const SumArgs<I, DT>& a, const Task& t,
       if (lane < n) {
         const int64_t at = a.dwperm ? static_cast<int64_t>(a.wperm ? my_wp : a.dwperm[base + lane])
                                     : base + lane;
-        a.dw[tile * a.dw_tile + at] = dw_stage[lane];
+        const float d = dw_stage[lane];
+        a.dw[tile * a.dw_tile + at] = d;
+        nan |= d != d;
       }
       __builtin_amdgcn_wave_barrier();
+    }
+  }
+  if constexpr (DW && VEC > 1) {
+    if (F % VEC != 0 && __any(nan)) {
+      const int64_t first = static_cast<int64_t>(tile) * (G * VEC);
+      redo_nan_dw(a, t.row, t.e0 + lane, t.e1, kWave, tile * a.dw_tile, first,
+                  first + G * VEC < F ? first + G * VEC : F);
     }
   }
   // Fold the EPW edge groups (lanes with equal c).
@@ -289,10 +322,10 @@ __device__ __forceinline__ void sum_task(const SumArgs<I, DT>& a, const Task& t,
     V::store(a.out + static_cast<int64_t>(t.row) * F + lc.at, acc);
 }
 
-template <typename I, int DT, int VEC, int G, int U>
+template <typename I, int DT, int VEC, int G, int U, bool DW>
 __global__ __launch_bounds__(kTaskBlock) void sum_rows_kernel(SumArgs<I, DT> a) {
   __shared__ float dw_stage[kWavesPerBlock][kWave];
-  sum_task<I, DT, VEC, G, U>(a, decode_task(a.plan, a.row_ptr, global_wave()), blockIdx.y,
+  sum_task<I, DT, VEC, G, U, DW>(a, decode_task(a.plan, a.row_ptr, global_wave()), blockIdx.y,
                              dw_stage[threadIdx.x / kWave]);
 }
 
@@ -308,7 +341,7 @@ __global__ __launch_bounds__(kTaskBlock) void sum_rows_kernel(SumArgs<I, DT> a) 
 template <int SLOT>
 constexpr int kSlotRow = 4 * SLOT;
 
-template <typename I, int DT, int VEC, int G, int UC, int SLOT, int P, int U>
+template <typename I, int DT, int VEC, int G, int UC, int SLOT, int P, int U, bool DW>
 __global__ __launch_bounds__(kTaskBlock) void sum_pairs_kernel(SumArgs<I, DT> a) {
   typedef Vec<VEC, DT> V;
   constexpr int NS = kWave / SLOT;   // slots per wave
@@ -321,7 +354,7 @@ __global__ __launch_bounds__(kTaskBlock) void sum_pairs_kernel(SumArgs<I, DT> a)
   const int64_t n_groups = (p.n_wave + NS * P - 1) / (NS * P);
   const int64_t pw = w - p.n_chunks;
   if (pw < 0 || pw >= n_groups) {
-    sum_task<I, DT, VEC, G, UC>(
+    sum_task<I, DT, VEC, G, UC, DW>(
         a, decode_task(p, a.row_ptr, pw < 0 ? w : p.n_chunks + p.n_wave + (pw - n_groups)), 0,
         stage);
     return;
@@ -331,7 +364,6 @@ __global__ __launch_bounds__(kTaskBlock) void sum_pairs_kernel(SumArgs<I, DT> a)
   const int g = hl / G, c = hl % G;
   const int64_t F = a.F;
   const LaneCols lc = lane_cols<VEC>(c * VEC, F);   // (one tile)
-  const bool want_dw = a.self_x != nullptr;
   int row[P], len[P];
   int64_t e0[P];
   bool has[P];      // rows the slots sum here
@@ -357,9 +389,10 @@ __global__ __launch_bounds__(kTaskBlock) void sum_pairs_kernel(SumArgs<I, DT> a)
   for (int m = SLOT; m < kWave; m <<= 1) len_max = max(len_max, __shfl_xor(len_max, m, 64));
   len_max = uniform(len_max);
   float self[P][VEC] = {}, acc[P][VEC] = {};
+  bool nan = false;
 #pragma unroll
   for (int q = 0; q < P; ++q)
-    if (want_dw && lc.active && has[q])
+    if (DW && lc.active && has[q])
       load_self<VEC, DT>(a.self_x + static_cast<int64_t>(row[q]) * F, lc, self[q]);
   for (int base = 0; base < len_max; base += SLOT) {
     int n[P], my_col[P], my_wp[P];
@@ -405,13 +438,13 @@ __global__ __launch_bounds__(kTaskBlock) void sum_pairs_kernel(SumArgs<I, DT> a)
 #pragma unroll
             for (int r = 0; r < VEC; ++r) acc[q][r] += wt[q][u] * f[r];
           }
-          if (want_dw) {
+          if constexpr (DW) {
             const float d = group_sum<G>(dot(f, self[q]));
             if (c == 0 && slot[u] < n[q]) stage[q * kWave + SLOT * slot_id + slot[u]] = d;
           }
         }
     }
-    if (want_dw) {
+    if constexpr (DW) {
       // (As in sum_task: dw leaves after the window, one store per lane.)
       __builtin_amdgcn_wave_barrier();
 #pragma unroll
@@ -419,9 +452,18 @@ __global__ __launch_bounds__(kTaskBlock) void sum_pairs_kernel(SumArgs<I, DT> a)
         if (hl < n[q]) {
           const int64_t e = e0[q] + base + hl;
           const int64_t at = a.dwperm ? static_cast<int64_t>(a.wperm ? my_wp[q] : a.dwperm[e]) : e;
-          a.dw[at] = stage[q * kWave + lane];
+          const float d = stage[q * kWave + lane];
+          a.dw[at] = d;
+          nan |= d != d;
         }
       __builtin_amdgcn_wave_barrier();
+    }
+  }
+  if constexpr (DW && VEC > 1) {
+    if (F % VEC != 0 && __any(nan)) {
+#pragma unroll
+      for (int q = 0; q < P; ++q)
+        redo_nan_dw(a, row[q], e0[q] + hl, e0[q] + len[q], SLOT, 0, 0, F);
     }
   }
   // Fold each row's edge groups (lanes with equal c; masks below SLOT stay
@@ -439,7 +481,7 @@ __global__ __launch_bounds__(kTaskBlock) void sum_pairs_kernel(SumArgs<I, DT> a)
   for (int q = 0; q < P; ++q)
     for (uint64_t m = late[q]; m; m &= m - 1) {
       const int64_t k = NS * P * pw + NS * q + (__ffsll(static_cast<long long>(m)) - 1) / SLOT;
-      sum_task<I, DT, VEC, G, UC>(a, decode_task(p, a.row_ptr, p.n_chunks + k), 0, stage);
+      sum_task<I, DT, VEC, G, UC, DW>(a, decode_task(p, a.row_ptr, p.n_chunks + k), 0, stage);
     }
 }
 
@@ -478,12 +520,15 @@ void launch_sum(const SumArgs<I, DT>& a, int tiles, hipStream_t s) {
     constexpr int US = G < 8 ? G : 8;
     const int64_t waves = p.n_chunks + (p.n_wave + NS * P - 1) / (NS * P) +
                           (p.n_empty + kEmptyPerWave - 1) / kEmptyPerWave;
-    sum_pairs_kernel<I, DT, VEC, G, U, SLOT, P, US>
-        <<<static_cast<unsigned>(ceil_div(waves, kWavesPerBlock)), kTaskBlock, 0, s>>>(a);
+    const auto k = a.self_x ? sum_pairs_kernel<I, DT, VEC, G, U, SLOT, P, US, true>
+                            : sum_pairs_kernel<I, DT, VEC, G, U, SLOT, P, US, false>;
+    k<<<static_cast<unsigned>(ceil_div(waves, kWavesPerBlock)), kTaskBlock, 0, s>>>(a);
   } else {
     const dim3 grid(static_cast<unsigned>(ceil_div(plan_waves(p), kWavesPerBlock)),
                     static_cast<unsigned>(tiles));
-    sum_rows_kernel<I, DT, VEC, G, U><<<grid, kTaskBlock, 0, s>>>(a);
+    const auto k = a.self_x ? sum_rows_kernel<I, DT, VEC, G, U, true>
+                            : sum_rows_kernel<I, DT, VEC, G, U, false>;
+    k<<<grid, kTaskBlock, 0, s>>>(a);
   }
 }
 
