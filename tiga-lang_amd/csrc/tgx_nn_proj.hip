@@ -562,7 +562,11 @@ __global__ __launch_bounds__(256, ACT < 0 ? 3 : 4) void projected_bwd_kernel(
 
 // Destination rows: the sum of dz (partial sums added in edge order), its
 // fields' gradient W1_dst^T (sum dz), and the sums (sum dz) (x) x_dst on MFMA.
-// A 16-lane group per row, lane hh holding hidden unit hh.
+// A 16-lane group per row, lane hh holding hidden unit hh.  A row over more than
+// kOwnPartials waves of edges is summed by the workgroup's 16 groups, every 16th
+// partial sum each (a hub of a million edges has 16,000: backward 3.57 ms with
+// one group walking them, 0.23 so).
+constexpr int kRowGroups = 16, kOwnPartials = 16;
 template <typename I>
 __global__ __launch_bounds__(256) void projected_rows_kernel(const I* __restrict__ row_ptr,
                                                              int64_t n_rows, ProjView v,
@@ -570,9 +574,12 @@ __global__ __launch_bounds__(256) void projected_rows_kernel(const I* __restrict
                                                              const float* __restrict__ part,
                                                              float* __restrict__ sums) {
   __shared__ float red[4][HP * kU];
+  __shared__ int range[kRowGroups][2];
+  __shared__ float fold[kRowGroups][HP];
   const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
   const int q = lane >> 4, hh = lane & 15;
+  const int group = threadIdx.x >> 4;
   float wt[HP];   // column hh of W1_dst
 #pragma unroll
   for (int h = 0; h < HP; ++h) wt[h] = v.packed[Packed::wt + hh * HP + h];
@@ -590,25 +597,52 @@ __global__ __launch_bounds__(256) void projected_rows_kernel(const I* __restrict
       grad = v.dst.f[s].grad + hh - v.dst.f[s].off;
     }
   f32x4m acc{0.f, 0.f, 0.f, 0.f};
-  const int64_t step = static_cast<int64_t>(gridDim.x) * 16;
-  for (int64_t first = static_cast<int64_t>(blockIdx.x) * 16 + wave * 4; first < n_rows;
+  const int64_t step = static_cast<int64_t>(gridDim.x) * kRowGroups;
+  for (int64_t first = static_cast<int64_t>(blockIdx.x) * kRowGroups; first < n_rows;
        first += step) {
-    const int64_t row = first + q;
+    const int64_t row = first + group;
     const bool valid = row < n_rows;
     const int64_t r0 = valid ? row_ptr[row] : 0, r1 = valid ? row_ptr[row + 1] : 0;
     // A row without edges has no part in the layer: its fields are not read
     // (they may be Inf or NaN, a mean over no neighbours) and its gradient is 0.
     const bool any = r1 > r0;
+    const int64_t w0 = r0 / kWave, w1 = any ? (r1 - 1) / kWave : w0;
+    const bool shared = w1 - w0 > kOwnPartials;
     float dz = 0.f, u = 0.f;
     if (any) {
-      const int64_t w0 = r0 / kWave, w1 = (r1 - 1) / kWave;
       if (w0 == w1) {
         dz = dzt[row * HP + hh];
-      } else {
+      } else if (!shared) {
         dz = part[(w0 * 2 + 1) * HP + hh];
         for (int64_t w = w0 + 1; w <= w1; ++w) dz += part[w * 2 * HP + hh];
       }
       if (x) u = x[row * stride];
+    }
+    if (__syncthreads_or(shared)) {
+      if (hh == 0) {   // (Below 2^31 edges: a wave's index fits.)
+        range[group][0] = static_cast<int>(w0);
+        range[group][1] = static_cast<int>(shared ? w1 : w0);
+      }
+      __syncthreads();
+      for (int k = 0; k < kRowGroups; ++k) {
+        const int64_t a = range[k][0], b = range[k][1];
+        if (a == b) continue;
+        float s = group == 0 ? part[(a * 2 + 1) * HP + hh] : 0.f;
+        int64_t w = a + 1 + group;
+        for (; w + 7 * kRowGroups <= b; w += 8 * kRowGroups) {
+          float y[8];
+#pragma unroll
+          for (int r = 0; r < 8; ++r) y[r] = part[(w + r * kRowGroups) * 2 * HP + hh];
+#pragma unroll
+          for (int r = 0; r < 8; ++r) s += y[r];
+        }
+        for (; w <= b; w += kRowGroups) s += part[w * 2 * HP + hh];
+        fold[group][hh] = s;
+        __syncthreads();
+        if (group == k)
+          for (int r = 0; r < kRowGroups; ++r) dz += fold[r][hh];
+        __syncthreads();
+      }
     }
     float g = 0.f;
 #pragma unroll
