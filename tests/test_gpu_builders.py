@@ -191,3 +191,55 @@ def test_from_coo_range_checks_and_strided_edge_lists(dtype):
         with pytest.raises(ValueError, match=f"{name} contains an out-of-range"):
             tg.Graph.from_coo(torch.tensor(src, dtype=dtype, device=DEV),
                               torch.tensor(dst, dtype=dtype, device=DEV), num_src=5, num_dst=4)
+
+
+# Empty rows inside a tile of 2048 edges, to both sides of the 20480 rows from
+# which a tile's edges search for their rows: between two of its edges, before
+# the first, after the last, at a tile's end, and all over.
+@pytest.mark.parametrize("n_rows,at", [
+    (20_481, [0, 20_480]), (20_482, [0, 20_481]), (22_528, [4096] * 2048), (30_000, [29_999]),
+    (30_000, [0, 0, 0]), (1_000_000, [7] * 2047 + [900_000] * 2 + [999_999]),
+    (300_000, list(range(0, 300_000, 101))), (40_000, [5] * 2048 + [39_990] * 2048),
+])
+@pytest.mark.parametrize("row_bits,out_bits", [(32, 32), (64, 64), (64, 32), (32, 64)])
+def test_destination_index_over_gaps(n_rows, at, row_bits, out_bits):
+    print(f"destination index gaps rows={n_rows} edges={len(at)}", flush=True)
+    ints = {32: torch.int32, 64: torch.int64}
+    rows = torch.tensor(at, device=DEV)
+    row_ptr = torch.zeros(n_rows + 1, dtype=torch.int64, device=DEV)
+    row_ptr[1:] = torch.cumsum(torch.bincount(rows, minlength=n_rows), 0)
+    row_ptr = row_ptr.to(ints[row_bits])
+    out = torch.full((len(at) + 1,), -7, dtype=ints[out_bits], device=DEV)
+    _native.call("tgx_destination_index", row_ptr.data_ptr(), row_bits, n_rows, len(at),
+                 out.data_ptr(), out_bits, _native.stream_of(out))
+    assert torch.equal(out[:-1].long(), rows) and int(out[-1]) == -7
+
+
+def test_destination_index_does_not_walk_gaps():
+    """Four million empty rows between two edges of one tile take no longer than
+    the same rows of 4 edges each (walked by one workgroup: over ten times)."""
+    print("destination index gap time", flush=True)
+    n_rows = 4_000_000
+    times = []
+    for gap in (False, True):
+        degree = torch.zeros(n_rows, dtype=torch.int64, device=DEV)
+        if gap:
+            degree[0] = degree[-1] = 2_000
+        else:
+            degree += 4
+        row_ptr = torch.zeros(n_rows + 1, dtype=torch.int64, device=DEV)
+        row_ptr[1:] = torch.cumsum(degree, 0)
+        E = int(row_ptr[-1])
+        out = torch.empty(E, dtype=torch.int64, device=DEV)
+        best = float("inf")
+        for _ in range(10):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            _native.call("tgx_destination_index", row_ptr.data_ptr(), 64, n_rows, E,
+                         out.data_ptr(), 64, _native.stream_of(out))
+            end.record()
+            end.synchronize()
+            best = min(best, start.elapsed_time(end))
+        times.append(best)
+    print("   16M edges, 4,000 edges about a gap, ms:", times, flush=True)
+    assert times[1] <= 2 * times[0]
