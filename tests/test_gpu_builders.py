@@ -243,3 +243,19 @@ def test_destination_index_does_not_walk_gaps():
         times.append(best)
     print("   16M edges, 4,000 edges about a gap, ms:", times, flush=True)
     assert times[1] <= 2 * times[0]
+
+
+def test_destination_index_of_more_rows_than_int32():
+    """64-bit row ids past 2^31 - 1 rows; 32-bit ones are refused."""
+    print("destination index past 2^31 rows", flush=True)
+    n_rows = 2**31 + 5
+    row_ptr = torch.zeros(n_rows + 1, dtype=torch.int64, device=DEV)
+    row_ptr[-2:] = torch.tensor([2, 5], device=DEV)
+    out = torch.empty(5, dtype=torch.int64, device=DEV)
+    args = (row_ptr.data_ptr(), 64, n_rows, 5, out.data_ptr())
+    _native.call("tgx_destination_index", *args, 64, _native.stream_of(out))
+    assert out.tolist() == [n_rows - 2] * 2 + [n_rows - 1] * 3
+    with pytest.raises(RuntimeError, match="row ids overflow int32"):
+        _native.call("tgx_destination_index", *args, 32, _native.stream_of(out))
+    del row_ptr
+    torch.cuda.empty_cache()

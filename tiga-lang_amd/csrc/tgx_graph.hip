@@ -690,7 +690,7 @@ extern "C" int tgx_destination_index(const void* row_ptr, int idx_bits, int64_t 
   TGX_REQUIRE(n_rows >= 0 && n_edges >= 0, "negative size");
   if (n_rows == 0 || n_edges == 0) return TGX_OK;
   TGX_REQUIRE(row_ptr && out, "null pointer");
-  TGX_REQUIRE(n_rows <= INT32_MAX, "row ids overflow int32");
+  TGX_REQUIRE(out_bits == 64 || n_rows <= INT32_MAX, "row ids overflow int32");
   hipStream_t s = as_stream(stream);
   const auto run = [&](const auto* rp, auto* o) {
     destination_index_kernel<<<ceil_div(n_edges, kIndexTile), kBlock, 0, s>>>(rp, n_rows, n_edges,
