@@ -105,14 +105,22 @@ int tgx_coo_to_csr_workspace(int64_t n_src, int64_t n_dst, int64_t n_edges,
  *   row_ptr_dev [n_dst+1] in dst's width (dst_bits)
  *   col_dev     [n_edges] in src's width (src_bits): src in stable dst order
  *   perm_dev    [n_edges] int32: argsort(dst, stable=True); may be NULL
- * Every dst must lie in [0, n_dst).  Supports n_edges, n_dst < 2^31.
- * n_src > 0 says that every src lies in [0, n_src): 64-bit sources below
- * 2^31 then move as 32-bit values; 0 says nothing about them.
+ * Every dst must lie in [0, n_dst); sources are moved as they are, whatever
+ * n_src is.  Supports n_edges, n_dst < 2^31.
  * Deterministic: output is bit-identical across runs. */
 int tgx_coo_to_csr(const void* src_dev, int src_bits, const void* dst_dev,
                    int dst_bits, int64_t n_src, int64_t n_dst, int64_t n_edges,
                    void* row_ptr_dev, void* col_dev, int32_t* perm_dev,
                    void* workspace_dev, size_t workspace_bytes, void* stream);
+
+/* tgx_coo_to_csr where every src is known to lie in [0, n_src): 64-bit sources
+ * of n_src <= 2^31 then move as 32-bit values through the sort (a source
+ * outside would be cut), instead of being gathered after it.  The workspace is
+ * tgx_coo_to_csr_workspace's. */
+int tgx_coo_to_csr_in_range(const void* src_dev, int src_bits, const void* dst_dev,
+                            int dst_bits, int64_t n_src, int64_t n_dst, int64_t n_edges,
+                            void* row_ptr_dev, void* col_dev, int32_t* perm_dev,
+                            void* workspace_dev, size_t workspace_bytes, void* stream);
 
 /* Workspace bytes needed by tgx_varlen_csr. */
 int tgx_varlen_csr_workspace(int64_t n_seq, size_t* bytes);

@@ -259,3 +259,35 @@ def test_destination_index_of_more_rows_than_int32():
         _native.call("tgx_destination_index", *args, 32, _native.stream_of(out))
     del row_ptr
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("n_rows,n_edges", [(1, 3), (2048, 8193), ((1 << 22) + 1, 20_000)])
+@pytest.mark.parametrize("src_bits", [32, 64])
+def test_coo_sources_are_moved_as_they_are(n_rows, n_edges, src_bits):
+    """tgx_coo_to_csr takes its n_src for nothing: any source, 64-bit ones past
+    2^31 and negative ones among them, arrives whole.  tgx_coo_to_csr_in_range
+    gives the same for sources in range."""
+    print(f"coo sources rows={n_rows} edges={n_edges} {src_bits}", flush=True)
+    ints = {32: torch.int32, 64: torch.int64}
+    g = torch.Generator(device=DEV).manual_seed(n_edges)
+    top = 2 ** (src_bits - 1) - 1
+    dst = torch.randint(0, n_rows, (n_edges,), device=DEV, generator=g)
+    order = torch.argsort(dst, stable=True)
+    ws_bytes = ctypes.c_size_t()
+    _native.call("tgx_coo_to_csr_workspace", 5, n_rows, n_edges, ctypes.byref(ws_bytes))
+    ws = torch.empty(ws_bytes.value, dtype=torch.uint8, device=DEV)
+    row_ptr = torch.empty(n_rows + 1, dtype=torch.int64, device=DEV)
+    for name, low, high, n_src in (("tgx_coo_to_csr", -top - 1, top, 5),
+                                   ("tgx_coo_to_csr", 0, 5, 0),
+                                   ("tgx_coo_to_csr_in_range", 0, 2**31 - 1, 2**31 - 1),
+                                   ("tgx_coo_to_csr_in_range", 0, top, top)):
+        src = torch.randint(low, high, (n_edges,), device=DEV, generator=g).to(ints[src_bits])
+        src[-1] = high - 1
+        for perm in (None, torch.empty(n_edges, dtype=torch.int32, device=DEV)):
+            col = torch.empty_like(src)
+            _native.call(name, src.data_ptr(), src_bits, dst.data_ptr(), 64, n_src, n_rows,
+                         n_edges, row_ptr.data_ptr(), col.data_ptr(),
+                         None if perm is None else perm.data_ptr(), ws.data_ptr(),
+                         ws_bytes.value, _native.stream_of(dst))
+            assert torch.equal(col, src[order])
+            assert perm is None or torch.equal(perm.long(), order)

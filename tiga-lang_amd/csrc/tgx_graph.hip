@@ -1032,18 +1032,17 @@ size_t coo_bytes(int64_t n_edges) {
 }
 
 template <typename S, typename D>
-int coo_impl(const S* src, const D* dst, int64_t n_src, int64_t n_dst, int64_t E, D* row_ptr,
+int coo_impl(const S* src, const D* dst, bool fits32, int64_t n_dst, int64_t E, D* row_ptr,
              S* col, int32_t* perm, void* ws, size_t ws_bytes, hipStream_t s) {
   const size_t need = coo_bytes(E);
   TGX_REQUIRE(ws_bytes >= need, "workspace too small: need %zu bytes", need);
   Carve c{static_cast<char*>(ws), ws_bytes};
   int st = TGX_OK;
   const uint32_t* sorted = nullptr;
-  // Sources that fit 32 bits (a 32-bit array, or the caller's promise that
-  // they are below n_src) ride through the sort as its payload; others are
-  // gathered through the permutation, a line of memory per edge (16.8M edges:
-  // 344 us for that gather).
-  const bool ride = sizeof(S) == 4 || (n_src > 0 && n_src <= (int64_t{1} << 31));
+  // Sources that fit 32 bits (a 32-bit array, or the caller's word for it) ride
+  // through the sort as its payload; others are gathered through the
+  // permutation, a line of memory per edge (16.8M edges: 344 us for that gather).
+  const bool ride = sizeof(S) == 4 || fits32;
   const SortColumn<int32_t, int32_t> order{nullptr, perm};
   if (ride) {
     sorted = stable_sort_by_key(dst, E, n_dst, SortColumn<S, S>{src, col}, order, c, s, &st);
@@ -1067,16 +1066,38 @@ int coo_impl(const S* src, const D* dst, int64_t n_src, int64_t n_dst, int64_t E
 }
 
 template <typename S>
-int coo_dispatch_dst(const S* src, const void* dst, int dst_bits, int64_t n_src, int64_t n_dst,
+int coo_dispatch_dst(const S* src, const void* dst, int dst_bits, bool fits32, int64_t n_dst,
                      int64_t E, void* row_ptr, void* col, int32_t* perm, void* ws,
                      size_t ws_bytes, hipStream_t s) {
   if (dst_bits == 32)
-    return coo_impl(src, static_cast<const int32_t*>(dst), n_src, n_dst, E,
+    return coo_impl(src, static_cast<const int32_t*>(dst), fits32, n_dst, E,
                     static_cast<int32_t*>(row_ptr), static_cast<S*>(col), perm, ws,
                     ws_bytes, s);
-  return coo_impl(src, static_cast<const int64_t*>(dst), n_src, n_dst, E,
+  return coo_impl(src, static_cast<const int64_t*>(dst), fits32, n_dst, E,
                   static_cast<int64_t*>(row_ptr), static_cast<S*>(col), perm, ws, ws_bytes,
                   s);
+}
+
+int coo_checked(const void* src, int src_bits, const void* dst, int dst_bits, bool fits32,
+                int64_t n_dst, int64_t n_edges, void* row_ptr, void* col, int32_t* perm, void* ws,
+                size_t ws_bytes, void* stream) {
+  TGX_REQUIRE(src_bits == 32 || src_bits == 64, "src_bits must be 32 or 64");
+  TGX_REQUIRE(dst_bits == 32 || dst_bits == 64, "dst_bits must be 32 or 64");
+  TGX_REQUIRE(n_dst >= 0 && n_edges >= 0, "negative size");
+  TGX_REQUIRE(n_edges <= INT32_MAX && n_dst < INT32_MAX,
+              "the device builder supports < 2^31 edges and destinations");
+  TGX_REQUIRE(row_ptr, "null row_ptr");
+  hipStream_t s = as_stream(stream);
+  if (n_edges == 0) {
+    TGX_HIP(hipMemsetAsync(row_ptr, 0, (dst_bits / 8) * (n_dst + 1), s));
+    return TGX_OK;
+  }
+  TGX_REQUIRE(src && dst && col && ws, "null pointer");
+  if (src_bits == 32)
+    return coo_dispatch_dst(static_cast<const int32_t*>(src), dst, dst_bits, fits32, n_dst,
+                            n_edges, row_ptr, col, perm, ws, ws_bytes, s);
+  return coo_dispatch_dst(static_cast<const int64_t*>(src), dst, dst_bits, fits32, n_dst, n_edges,
+                          row_ptr, col, perm, ws, ws_bytes, s);
 }
 
 size_t varlen_csr_bytes(int64_t n_seq) {
@@ -1124,23 +1145,18 @@ extern "C" int tgx_coo_to_csr(const void* src, int src_bits, const void* dst, in
                               int64_t n_src, int64_t n_dst, int64_t n_edges, void* row_ptr,
                               void* col, int32_t* perm, void* ws, size_t ws_bytes,
                               void* stream) {
-  TGX_REQUIRE(src_bits == 32 || src_bits == 64, "src_bits must be 32 or 64");
-  TGX_REQUIRE(dst_bits == 32 || dst_bits == 64, "dst_bits must be 32 or 64");
-  TGX_REQUIRE(n_src >= 0 && n_dst >= 0 && n_edges >= 0, "negative size");
-  TGX_REQUIRE(n_edges <= INT32_MAX && n_dst < INT32_MAX,
-              "the device builder supports < 2^31 edges and destinations");
-  TGX_REQUIRE(row_ptr, "null row_ptr");
-  hipStream_t s = as_stream(stream);
-  if (n_edges == 0) {
-    TGX_HIP(hipMemsetAsync(row_ptr, 0, (dst_bits / 8) * (n_dst + 1), s));
-    return TGX_OK;
-  }
-  TGX_REQUIRE(src && dst && col && ws, "null pointer");
-  if (src_bits == 32)
-    return coo_dispatch_dst(static_cast<const int32_t*>(src), dst, dst_bits, n_src, n_dst,
-                            n_edges, row_ptr, col, perm, ws, ws_bytes, s);
-  return coo_dispatch_dst(static_cast<const int64_t*>(src), dst, dst_bits, n_src, n_dst, n_edges,
-                          row_ptr, col, perm, ws, ws_bytes, s);
+  TGX_REQUIRE(n_src >= 0, "negative size");
+  return coo_checked(src, src_bits, dst, dst_bits, false, n_dst, n_edges, row_ptr, col, perm, ws,
+                     ws_bytes, stream);
+}
+
+extern "C" int tgx_coo_to_csr_in_range(const void* src, int src_bits, const void* dst,
+                                       int dst_bits, int64_t n_src, int64_t n_dst,
+                                       int64_t n_edges, void* row_ptr, void* col, int32_t* perm,
+                                       void* ws, size_t ws_bytes, void* stream) {
+  TGX_REQUIRE(n_src >= 0, "negative size");
+  return coo_checked(src, src_bits, dst, dst_bits, n_src <= (int64_t{1} << 31), n_dst, n_edges,
+                     row_ptr, col, perm, ws, ws_bytes, stream);
 }
 
 extern "C" int tgx_varlen_csr_workspace(int64_t n_seq, size_t* bytes) {

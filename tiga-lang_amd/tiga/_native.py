@@ -68,6 +68,8 @@ _SIGNATURES: dict[str, list] = {
     "tgx_coo_to_csr_workspace": [c_i64, c_i64, c_i64, P(c_size)],
     "tgx_coo_to_csr": [c_vp, c_int, c_vp, c_int, c_i64, c_i64, c_i64, c_vp, c_vp, c_vp,
                        c_vp, c_size, c_vp],
+    "tgx_coo_to_csr_in_range": [c_vp, c_int, c_vp, c_int, c_i64, c_i64, c_i64, c_vp, c_vp, c_vp,
+                                c_vp, c_size, c_vp],
     "tgx_varlen_csr_workspace": [c_i64, P(c_size)],
     "tgx_varlen_csr": [c_vp, c_int, c_i64, c_i64, c_i64, c_int, c_vp, c_vp, c_vp, c_size,
                        c_vp],

@@ -158,7 +158,8 @@ def build_coo_csr(src: torch.Tensor, dst: torch.Tensor, num_dst: int, num_src: i
     ws_bytes = ctypes.c_size_t()
     _native.call("tgx_coo_to_csr_workspace", num_src, num_dst, E, ctypes.byref(ws_bytes))
     ws = torch.empty(max(ws_bytes.value, 1), dtype=torch.uint8, device=device)
-    _native.call("tgx_coo_to_csr", _native.ptr(src), _native.idx_bits(src), _native.ptr(dst),
+    _native.call("tgx_coo_to_csr_in_range" if num_src > 0 else "tgx_coo_to_csr",
+                 _native.ptr(src), _native.idx_bits(src), _native.ptr(dst),
                  _native.idx_bits(dst), num_src, num_dst, E, row_ptr.data_ptr(), col.data_ptr(),
                  None, ws.data_ptr(), ws_bytes.value, _native.stream_of(dst))
     return row_ptr, col[:E]
