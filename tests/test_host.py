@@ -560,3 +560,16 @@ def test_cpu_varlen_csr_matches_the_oracle_with_empty_sequences(causal, idx):
     assert r.dtype == idx and c.dtype == idx
     assert r.tolist() == rp.tolist() and c.tolist() == col.tolist()
     assert g.num_edges == int(rp[-1])
+
+
+@pytest.mark.parametrize("n_edges", [1 << 20, 16_777_217, 2**31 - 1])
+def test_sort_workspaces_stay_within_four_words_an_edge(n_edges):
+    """Edge sorts keep two key buffers and one of each payload (the other is the
+    output) and the tiles' counts, a byte an edge: 17 bytes an edge, whichever
+    node counts, where an 8-bit sort with its own row ids took 20.5."""
+    lib = _native.lib()
+    size = ctypes.c_size_t()
+    for name in ("tgx_csr_transpose_workspace", "tgx_coo_to_csr_workspace"):
+        for n_src, n_dst in ((0, 0), (1, 1 << 30), (1 << 30, 1)):
+            assert getattr(lib, name)(n_src, n_dst, n_edges, ctypes.byref(size)) == 0
+            assert size.value <= 17.1 * n_edges, name

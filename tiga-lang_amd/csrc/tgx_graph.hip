@@ -729,32 +729,52 @@ extern "C" int tgx_index_range(const void* idx, int idx_bits, int64_t n, int64_t
 namespace {
 
 // Scratch of one stable sort of n keys with up to two payloads: two key
-// buffers, two of each payload, the tiles' digit counts and their segments.
-void carve_sort(Carve& c, int64_t n) {
+// buffers, one of each payload (a payload's passes go to and fro between it and
+// the output), the tiles' digit counts and their segments.
+struct SortScratch {
+  uint32_t* keys[2];
+  int32_t* tmp[2];
+  int32_t *counts, *segments, *digit_first;
+};
+
+SortScratch carve_sort(Carve& c, int64_t n) {
   const int64_t nblocks = ceil_div(n, kSortTile);
-  for (int k = 0; k < 6; ++k) c.take<uint32_t>(n);
-  c.take<int32_t>(nblocks << kSortMaxBits);
-  c.take<int32_t>((ceil_div(nblocks, kSortSegment) + 1) << kSortMaxBits);
+  const int64_t nseg = ceil_div(nblocks, kSortSegment);
+  SortScratch x;
+  for (auto& k : x.keys) k = c.take<uint32_t>(n);
+  for (auto& t : x.tmp) t = c.take<int32_t>(n);
+  x.counts = c.take<int32_t>(nblocks << kSortMaxBits);
+  x.segments = c.take<int32_t>((nseg + 1) << kSortMaxBits);
+  x.digit_first = x.segments + (nseg << kSortMaxBits);
+  return x;
+}
+
+int sort_bits(int64_t key_range) {
+  int bits = 0;
+  while (bits < 32 && (static_cast<int64_t>(1) << bits) < key_range) ++bits;
+  return bits;
+}
+int sort_passes(int64_t key_range) {
+  const int bits = sort_bits(key_range);
+  return bits == 0 ? 1 : static_cast<int>(ceil_div(bits, kSortMaxBits));
 }
 
 // Stable LSD radix sort of keys in [0, key_range): the payload columns follow
 // their keys from col.in (null: the key's index) to col.out; c1.out null
-// sorts one column.  Returns the buffer that holds the sorted keys.  Scratch
-// is carved from c in the order carve_sort lays it out.
+// sorts one column.  Pass p writes a payload to its output if an even number of
+// passes follow, else to x.tmp, so col.in may be the one that pass 0 does not
+// write.  Returns the buffer that holds the sorted keys.
 template <typename K, typename P0, typename O0, typename P1>
 uint32_t* stable_sort_by_key(const K* keys, int64_t n, int64_t key_range, SortColumn<P0, O0> c0,
-                             SortColumn<P1, int32_t> c1, Carve& c, hipStream_t s, int* status) {
+                             SortColumn<P1, int32_t> c1, const SortScratch& x, hipStream_t s,
+                             int* status) {
   const int nb = static_cast<int>(ceil_div(n, kSortTile));
   const int nseg = static_cast<int>(ceil_div(nb, kSortSegment));
-  uint32_t* kbuf[2] = {c.take<uint32_t>(n), c.take<uint32_t>(n)};
-  int32_t* buf0[2] = {c.take<int32_t>(n), c.take<int32_t>(n)};
-  int32_t* buf1[2] = {c.take<int32_t>(n), c.take<int32_t>(n)};
-  int32_t* counts = c.take<int32_t>(static_cast<size_t>(nb) << kSortMaxBits);
-  int32_t* segments = c.take<int32_t>(static_cast<size_t>(nseg + 1) << kSortMaxBits);
-  int32_t* digit_first = segments + (static_cast<size_t>(nseg) << kSortMaxBits);
-  int bits = 0;
-  while (bits < 32 && (static_cast<int64_t>(1) << bits) < key_range) ++bits;
-  const int passes = bits == 0 ? 1 : static_cast<int>(ceil_div(bits, kSortMaxBits));
+  int32_t* const counts = x.counts;
+  int32_t* const segments = x.segments;
+  int32_t* const digit_first = x.digit_first;
+  const int bits = sort_bits(key_range);
+  const int passes = sort_passes(key_range);
   *status = TGX_OK;
   int shift = 0;
   for (int p = 0; p < passes; ++p) {
@@ -765,8 +785,8 @@ uint32_t* stable_sort_by_key(const K* keys, int64_t n, int64_t key_range, SortCo
     if (rb < 6) rb = 6;
     const int digits = 1 << rb;
     const bool first = p == 0, last = p == passes - 1;
-    uint32_t* const kout = kbuf[p % 2];
-    const uint32_t* const kin = first ? nullptr : kbuf[(p - 1) % 2];
+    uint32_t* const kout = x.keys[p % 2];
+    const uint32_t* const kin = first ? nullptr : x.keys[(p - 1) % 2];
     if (first)
       radix_count_kernel<<<nb, kSortBlock, 0, s>>>(keys, n, shift, rb, counts);
     else
@@ -791,10 +811,13 @@ uint32_t* stable_sort_by_key(const K* keys, int64_t n, int64_t key_range, SortCo
       }
     };
     // The first pass reads the caller's arrays, the last writes them.
-    int32_t* const out1 = !c1.out ? nullptr : last ? c1.out : buf1[p % 2];
-    const int32_t* const in0 = first ? nullptr : buf0[(p - 1) % 2];
-    const int32_t* const in1 = first ? nullptr : buf1[(p - 1) % 2];
-    int32_t* const mid0 = buf0[p % 2];
+    // (A 64-bit output holds 32-bit values until the last pass.)
+    int32_t* const o0 = reinterpret_cast<int32_t*>(c0.out);
+    const bool to_out = (passes - 1 - p) % 2 == 0;
+    int32_t* const mid0 = to_out ? o0 : x.tmp[0];
+    int32_t* const out1 = !c1.out ? nullptr : to_out ? c1.out : x.tmp[1];
+    const int32_t* const in0 = to_out ? x.tmp[0] : o0;
+    const int32_t* const in1 = to_out ? x.tmp[1] : c1.out;
     if (first && last)
       scatter(keys, c0, c1);
     else if (first)
@@ -811,13 +834,12 @@ uint32_t* stable_sort_by_key(const K* keys, int64_t n, int64_t key_range, SortCo
     }
     shift += rb;
   }
-  return kbuf[(passes - 1) % 2];
+  return x.keys[(passes - 1) % 2];
 }
 
 size_t transpose_bytes(int64_t n_edges) {
   Carve c{nullptr, 0};
   carve_sort(c, n_edges);
-  c.take<int32_t>(n_edges);  // destination row per edge
   return align_up(c.used);
 }
 
@@ -840,16 +862,16 @@ static int transpose_impl(const I* row_ptr, const I* col, int64_t n_dst, int64_t
   TGX_REQUIRE(ws_bytes >= need, "workspace too small: need %zu bytes", need);
   Carve c{static_cast<char*>(ws), ws_bytes};
   int st = TGX_OK;
+  const SortScratch x = carve_sort(c, E);
   // Each edge's destination row rides through the sort beside its index (a
-  // gather of it through perm afterwards would fetch a line per edge).
-  Carve after = c;
-  carve_sort(after, E);
-  int32_t* erow = after.take<int32_t>(E);
+  // gather of it through perm afterwards would fetch a line per edge), from the
+  // buffer that pass 0 leaves alone.
+  int32_t* const erow = sort_passes(n_src) % 2 ? x.tmp[1] : col_t;
   destination_index_kernel<<<ceil_div(E, kIndexTile), kBlock, 0, s>>>(row_ptr, n_dst, E, erow);
   TGX_LAUNCHED("destination_index_kernel");
   const uint32_t* sorted =
       stable_sort_by_key(col, E, n_src, SortColumn<int32_t, int32_t>{nullptr, perm},
-                         SortColumn<int32_t, int32_t>{erow, col_t}, c, s, &st);
+                         SortColumn<int32_t, int32_t>{erow, col_t}, x, s, &st);
   if (st != TGX_OK) return st;
   // row_ptr_t = lower bound of every source id in [0, n_src].
   run_end_fill_kernel<int32_t><<<ceil_div(n_src + 1, kBlock), kBlock, 0, s>>>(
@@ -1027,7 +1049,6 @@ namespace {
 size_t coo_bytes(int64_t n_edges) {
   Carve c{nullptr, 0};
   carve_sort(c, n_edges);
-  c.take<int32_t>(n_edges);  // permutation when the caller does not want it
   return align_up(c.used);
 }
 
@@ -1043,16 +1064,14 @@ int coo_impl(const S* src, const D* dst, bool fits32, int64_t n_dst, int64_t E, 
   // through the sort as its payload; others are gathered through the
   // permutation, a line of memory per edge (16.8M edges: 344 us for that gather).
   const bool ride = sizeof(S) == 4 || fits32;
+  const SortScratch x = carve_sort(c, E);
   const SortColumn<int32_t, int32_t> order{nullptr, perm};
   if (ride) {
-    sorted = stable_sort_by_key(dst, E, n_dst, SortColumn<S, S>{src, col}, order, c, s, &st);
+    sorted = stable_sort_by_key(dst, E, n_dst, SortColumn<S, S>{src, col}, order, x, s, &st);
   } else {
-    Carve after = c;
-    carve_sort(after, E);
-    int32_t* own_perm = after.take<int32_t>(E);
-    if (!perm) perm = own_perm;
+    if (!perm) perm = x.tmp[1];   // (one payload: free)
     sorted = stable_sort_by_key(dst, E, n_dst, SortColumn<int32_t, int32_t>{nullptr, perm},
-                                SortColumn<int32_t, int32_t>{nullptr, nullptr}, c, s, &st);
+                                SortColumn<int32_t, int32_t>{nullptr, nullptr}, x, s, &st);
   }
   if (st != TGX_OK) return st;
   run_end_fill_kernel<D><<<ceil_div(n_dst + 1, kBlock), kBlock, 0, s>>>(sorted, E, n_dst,
