@@ -314,6 +314,35 @@ def test_edge_weight_gradients_of_infinite_values(F_, dtype):
                 RTOL32 * float(want[finite].abs().max())
 
 
+def test_wide_edge_weight_gradient_without_its_workspace(monkeypatch):
+    """The workspace of a wide dw is a matter of speed: where it cannot be
+    allocated the backward runs without it."""
+    print("wide dw without workspace", flush=True)
+    rp, col = skewed_csr(3, 400, 300, mean_deg=5, hubs=(700,))
+    graph = tg.Graph.from_csr(to_dev(rp, torch.int64), to_dev(col, torch.int64), num_src=300)
+    g = torch.Generator(device=DEV).manual_seed(3)
+    x = torch.randn(300, 600, device=DEV, generator=g).requires_grad_(True)
+    w = torch.rand(col.size, device=DEV, generator=g).requires_grad_(True)
+    dout = torch.randn(400, 600, device=DEV, generator=g)
+    from tiga._ops import CsrSumFunction
+
+    out = CsrSumFunction.apply(x, w, graph)
+    want = torch.autograd.grad(out, (x, w), dout, retain_graph=True)
+    empty, refused = torch.empty, []
+
+    def scarce(*args, **kwargs):
+        if kwargs.get("dtype") is torch.uint8:
+            refused.append(args)
+            raise torch.OutOfMemoryError("no memory for scratch")
+        return empty(*args, **kwargs)
+
+    monkeypatch.setattr(torch, "empty", scarce)
+    got = torch.autograd.grad(out, (x, w), dout)
+    monkeypatch.undo()
+    assert len(refused) == 1 and torch.equal(got[0], want[0])
+    assert float((got[1] - want[1]).abs().max()) <= RTOL32 * float(want[1].abs().max())
+
+
 # ---- GAT additive ----------------------------------------------------------
 
 class GAT(tg.MessagePassing):

@@ -156,8 +156,11 @@ class CsrSumFunction(torch.autograd.Function):
                 _native.call("tgx_csr_sum_bwd_workspace", E, ctx.F, code,
                              ctypes.byref(ws_bytes))
                 ws_size = ws_bytes.value
-                if ws_size:
-                    ws = torch.empty(ws_size, dtype=torch.uint8, device=xc.device)
+                try:
+                    if ws_size:
+                        ws = torch.empty(ws_size, dtype=torch.uint8, device=xc.device)
+                except torch.OutOfMemoryError:
+                    ws_size = 0   # dw in a pass of its own, which needs none
             _native.call("tgx_csr_sum_bwd_ws", t.row_ptr_t.data_ptr(), t.col_t.data_ptr(),
                          t.perm.data_ptr(), t.plan.ref, xc.data_ptr(), _p(wc),
                          dout.data_ptr(), _p(dx), None if dw_in_csr else _p(dw), n_dst,
