@@ -311,6 +311,16 @@ int tgx_gat_fwd(const void* row_ptr_dev, const void* col_dev, int idx_bits,
                 int64_t n_dst, int64_t n_src, int H, int D, int dtype, float* partial_dev,
                 float* pos_dev, void* stream);
 
+/* tgx_gat_fwd for a relation of n_edges edges (0: not known, as tgx_gat_fwd):
+ * the same results; large fp32 tables with enough edges a row are gathered one
+ * half of the heads after the other. */
+int tgx_gat_fwd_edges(const void* row_ptr_dev, const void* col_dev, int idx_bits,
+                      const tgx_row_plan* plan, const void* h_src_dev, const void* h_dst_dev,
+                      const float* a_src_dev, const float* a_dst_dev,
+                      float negative_slope, void* out_dev, float* node_state_dev,
+                      int64_t n_dst, int64_t n_src, int64_t n_edges, int H, int D, int dtype,
+                      float* partial_dev, float* pos_dev, void* stream);
+
 /* Workspace bytes for tgx_gat_bwd with these plans and element type;
  * folded != 0 for a backward given the forward's pos (it needs no per-edge
  * buffer). */

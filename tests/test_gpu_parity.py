@@ -455,9 +455,8 @@ def test_gat_element_types_and_bipartite_parity(H, D, dtype, bipartite, a_typed)
     assert rel_err(f(a_d.grad), e_dad) <= a_tol
 
 
-# Tables of over 512 MB run the gathers one half of the heads after the other:
-# the last table that does not and the first that does (1 KB rows), and heads
-# that fill a lane group (nothing to halve).
+# Tables of half a GB of 1 KB rows with a tenth of an edge a row, which run whole,
+# and heads that fill a lane group (nothing to halve).
 @pytest.mark.parametrize("n_src,H,D", [(524_288, 8, 32), (524_289, 8, 32), (524_289, 2, 128),
                                        (524_289, 1, 256), (524_289, 3, 128)])
 @pytest.mark.parametrize("bipartite", [False, True])
@@ -499,6 +498,49 @@ def test_gat_halved_head_groups(n_src, H, D, bipartite):
                                      else [h64, as64, ad64], dout.double())
     for got, exp in zip([out.detach(), *grads], [want.detach(), *want_grads]):
         assert float((got.double() - exp).abs().max() / exp.abs().max()) <= RTOL32
+
+
+# 1 KB rows of tables over 768 MB with 12 edges a row or more run the forward one
+# half of the heads after the other, and up to 1536 MB the backward's source
+# pass too: sizes on both sides of each line, and bipartite relations that halve
+# one of the two.
+@pytest.mark.parametrize("n_dst,n_src,degree,halved", [
+    (786_433, 786_433, 12, (True, True)), (786_432, 786_432, 12, (False, False)),
+    (786_433, 786_433, 11, (False, False)), (1_572_865, 1_572_865, 12, (True, False)),
+    (100_000, 800_000, 12, (True, False)), (800_000, 50_000, 2, (False, True))])
+@pytest.mark.parametrize("H,D", [(8, 32), (2, 128)])
+def test_gat_halves_heads_where_edges_pay_for_it(n_dst, n_src, degree, halved, H, D):
+    """The rule's choices by the kernels' launches, and the results against
+    layers of each half of the heads, which are never halved: to the bit where
+    the halves run the same kernels, else up to the edge order of fp32 sums."""
+    print(f"gat halving {n_dst}x{n_src} degree={degree} H={H} D={D}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(degree)
+    cols = torch.randint(0, n_src, (n_dst * degree,), device=DEV, generator=g)
+    row_ptr = torch.arange(n_dst + 1, device=DEV) * degree
+    graph = tg.Graph.from_csr(row_ptr, cols, num_src=n_src)
+    homogeneous = n_dst == n_src
+    h = torch.randn(n_src, H, D, device=DEV, generator=g)
+    hd = h if homogeneous else torch.randn(n_dst, H, D, device=DEV, generator=g)
+    a_s, a_d = (0.1 * torch.randn(H, D, device=DEV, generator=g) for _ in range(2))
+    dout = torch.randn(n_dst, H, D, device=DEV, generator=g)
+
+    def layer(part):
+        x = h[:, part].contiguous().requires_grad_(True)
+        y = x if homogeneous else hd[:, part].contiguous().requires_grad_(True)
+        with _native.KernelTimer() as timer:
+            out = GAT(a_s[part], a_d[part], 0.2)(graph=graph, src={"h": x}, dst={"h": y})
+            grads = torch.autograd.grad(out, [x] if homogeneous else [x, y],
+                                        dout[:, part].contiguous())
+        return [out.detach(), *grads], timer.totals
+
+    whole, totals = layer(slice(None))
+    launches = [totals[k][0] for k in ("gat_fwd_kernel", "gat_bwd_src_kernel")]
+    assert launches == [2 if x else 1 for x in halved]
+    for part in (slice(0, H // 2), slice(H // 2, H)):
+        for k, (a, b) in enumerate(zip(whole, layer(part)[0])):
+            if halved[min(k, 1)] and halved[0]:
+                assert torch.equal(a[:, part], b)
+            assert float((a[:, part] - b).abs().max()) <= RTOL32 * float(b.abs().max())
 
 
 def test_gat_large_scores_and_determinism():

@@ -819,23 +819,35 @@ struct GatBwdIo {
   void *dhs, *dhd;
   float *ns, *da_src, *da_dst;
   const float* pos;  // the forward's folded destination rows, or null
-  int64_t n_dst, n_src, ld, nsld;
+  int64_t n_dst, n_src, n_edges, ld, nsld;
   float slope;
   int64_t col_off;   // the head group's first column (h0 * D) within a row
 };
 
-// fp32 rows of 1 KB (64 lanes) of a table over twice the Infinity Cache (256
-// MB): the gather passes run one half of the heads after the other.  Each pass
-// then gathers 512 bytes a row from half the bytes, twice as much of which the
-// cache holds, and its lines come at the L2s' rate (7 TB/s) where whole rows
-// wait for HBM (6.1 TB/s).  1M nodes, 17M edges, 8 heads of 32: forward 3.19 ->
-// 2.76 ms, source pass 3.56 -> 3.37 ms, edges read twice.  Quarters: 3.33 and
-// 4.22 ms; tables of 512 MB and less gain nothing (random rows alone: 500,000
-// of 1 KB 7.1 TB/s whole, 6.9 halved).
+// fp32 rows of 1 KB (64 lanes) of a table over three times the Infinity Cache
+// (256 MB): the gather passes run one half of the heads after the other where
+// there are 12 edges a row or more.  Each pass then gathers 512 bytes a row from
+// half the bytes, twice as much of which the cache holds, and its lines come
+// nearer the L2s' rate (7 TB/s) where whole rows wait for HBM (6.1 TB/s); the
+// rows' own work and the edges' columns come twice, so few edges lose.  8 heads
+// of 32, edges a row, whole -> halved us:
+//   forward, 1M rows    7: 1607 -> 1808   12: 2412 -> 2298   17: 3327 -> 2812
+//            0.7M rows 11: 1452 -> 1556   17: 2073 -> 1932   29: 3369 -> 3272
+//            0.8M rows 12: 1832 -> 1834   17: 2513 -> 2198
+//            3M rows   12: 8288 -> 8054   17: 11212 -> 10826
+//   backward (its source pass), 1M rows 7: 2527 -> 2582  12: 3479 -> 3350
+// The source pass gathers dout rows and node state, a part of it that the cache
+// serves either way: past six times the cache its halves miss like the whole
+// (1.5M rows, 17 edges 6946 -> 6941, 2M 9502 -> 9679, 0.6M 2074 -> 2147).
 template <int DT, int G, int HL>
 constexpr bool can_halve = DT == TGX_DTYPE_F32 && G == 64 && HL <= G / 2;
-bool halve_heads(int64_t table_rows, int row_floats) {
-  return table_rows * row_floats * 4 > (int64_t{512} << 20);
+constexpr int64_t kHalveTable = int64_t{768} << 20, kHalveEdges = 12;
+inline bool halve_fwd(int64_t n_src, int row_floats, int64_t n_edges, int64_t n_dst) {
+  return n_src * row_floats * 4 > kHalveTable && n_edges >= kHalveEdges * n_dst;
+}
+inline bool halve_bwd(int64_t n_dst, int row_floats, int64_t n_edges, int64_t n_src) {
+  const int64_t table = n_dst * row_floats * 4;
+  return table > kHalveTable && table <= 2 * kHalveTable && n_edges >= kHalveEdges * n_src;
 }
 
 // Node-pass grid: one wave per EPW nodes, at most what stays resident.
@@ -920,7 +932,7 @@ int gat_bwd_launch(const I* row_ptr, const tgx_row_plan& plan, const int32_t* ro
   };
   bool halves = false;
   if constexpr (can_halve<DT, G, HL>) {
-    if (folded && halve_heads(io.n_dst, HD)) {
+    if (folded && halve_bwd(io.n_dst, HD, io.n_edges, io.n_src)) {
       halves = true;
       for (int h : {0, G / HL / 2}) {
         const int st = src_pass(std::integral_constant<int, G / 2>{}, h);
@@ -1003,13 +1015,15 @@ int gat_bwd_launch(const I* row_ptr, const tgx_row_plan& plan, const int32_t* ro
 template <int DT>
 int gat_fwd_dtype(const void* row_ptr, const void* col, int idx_bits, const tgx_row_plan* plan,
                   const void* hs, const void* hd, const float* a_src, const float* a_dst,
-                  float slope, void* out, float* ns, int64_t n_src, int H, int D,
-                  float* partial, float* pos, hipStream_t s) {
+                  float slope, void* out, float* ns, int64_t n_dst, int64_t n_src,
+                  int64_t n_edges, int H, int D, float* partial, float* pos, hipStream_t s) {
   using T = typename Vals<DT, 4>::T;
   const int64_t ld = static_cast<int64_t>(H) * D, nsld = 4 * static_cast<int64_t>(H);
   for (int h0 = 0; h0 < H;) {
     int hg = gat_group_heads(H, D, h0);
-    if (DT == TGX_DTYPE_F32 && hg >= 2 && hg * D == 256 && halve_heads(n_src, hg * D)) hg /= 2;
+    if (DT == TGX_DTYPE_F32 && hg >= 2 && hg * D == 256 &&
+        halve_fwd(n_src, hg * D, n_edges, n_dst))
+      hg /= 2;
     const GatShape shp = gat_shape(hg, D);
     const int64_t off = static_cast<int64_t>(h0) * D;
     const T* hs_g = hs ? static_cast<const T*>(hs) + off : nullptr;
@@ -1101,11 +1115,11 @@ int gat_bwd_dtype(const void* row_ptr, int idx_bits, const tgx_row_plan* plan,
 
 using namespace tgx;
 
-extern "C" int tgx_gat_fwd(const void* row_ptr, const void* col, int idx_bits,
-                           const tgx_row_plan* plan, const void* h_src, const void* h_dst,
-                           const float* a_src, const float* a_dst, float slope, void* out,
-                           float* ns, int64_t n_dst, int64_t n_src, int H, int D, int dtype,
-                           float* partial, float* pos, void* stream) {
+extern "C" int tgx_gat_fwd_edges(const void* row_ptr, const void* col, int idx_bits,
+                                 const tgx_row_plan* plan, const void* h_src, const void* h_dst,
+                                 const float* a_src, const float* a_dst, float slope, void* out,
+                                 float* ns, int64_t n_dst, int64_t n_src, int64_t n_edges, int H,
+                                 int D, int dtype, float* partial, float* pos, void* stream) {
   TGX_REQUIRE(idx_bits == 32 || idx_bits == 64, "idx_bits must be 32 or 64");
   TGX_REQUIRE(dtype_bytes(dtype) != 0, "dtype must be TGX_DTYPE_BF16, _F16 or _F32 (got %d)",
               dtype);
@@ -1118,6 +1132,7 @@ extern "C" int tgx_gat_fwd(const void* row_ptr, const void* col, int idx_bits,
               "one feature tensor for both roles needs n_src == n_dst");
   int st = check_plan(plan, n_dst);
   if (st != TGX_OK) return st;
+  TGX_REQUIRE(n_edges >= 0, "negative edge count");
   if (n_dst == 0) return TGX_OK;
   TGX_REQUIRE(row_ptr && h_dst && a_src && a_dst && out && ns && (h_src || n_src == 0),
               "null pointer");
@@ -1128,14 +1143,26 @@ extern "C" int tgx_gat_fwd(const void* row_ptr, const void* col, int idx_bits,
   switch (dtype) {
     case TGX_DTYPE_F32:
       return gat_fwd_dtype<TGX_DTYPE_F32>(row_ptr, col, idx_bits, plan, h_src, h_dst, a_src,
-                                          a_dst, slope, out, ns, n_src, H, D, partial, pos, s);
+                                          a_dst, slope, out, ns, n_dst, n_src, n_edges, H, D, partial,
+                                          pos, s);
     case TGX_DTYPE_BF16:
       return gat_fwd_dtype<TGX_DTYPE_BF16>(row_ptr, col, idx_bits, plan, h_src, h_dst, a_src,
-                                           a_dst, slope, out, ns, n_src, H, D, partial, pos, s);
+                                           a_dst, slope, out, ns, n_dst, n_src, n_edges, H, D, partial,
+                                          pos, s);
     default:
       return gat_fwd_dtype<TGX_DTYPE_F16>(row_ptr, col, idx_bits, plan, h_src, h_dst, a_src,
-                                          a_dst, slope, out, ns, n_src, H, D, partial, pos, s);
+                                          a_dst, slope, out, ns, n_dst, n_src, n_edges, H, D, partial,
+                                          pos, s);
   }
+}
+
+extern "C" int tgx_gat_fwd(const void* row_ptr, const void* col, int idx_bits,
+                           const tgx_row_plan* plan, const void* h_src, const void* h_dst,
+                           const float* a_src, const float* a_dst, float slope, void* out,
+                           float* ns, int64_t n_dst, int64_t n_src, int H, int D, int dtype,
+                           float* partial, float* pos, void* stream) {
+  return tgx_gat_fwd_edges(row_ptr, col, idx_bits, plan, h_src, h_dst, a_src, a_dst, slope, out,
+                           ns, n_dst, n_src, 0, H, D, dtype, partial, pos, stream);
 }
 
 extern "C" int tgx_gat_bwd_workspace(const tgx_row_plan* plan, const tgx_row_plan* plan_t,
@@ -1198,8 +1225,8 @@ extern "C" int tgx_gat_bwd(const void* row_ptr, const void* col, int idx_bits,
   TGX_REQUIRE(ws && ws_bytes >= need, "workspace too small: need %zu bytes", need);
   hipStream_t s = as_stream(stream);
   const GatBwdIo io{h_src, h_dst, out, dout, a_src, a_dst, dh_src, dh_dst, ns, da_src, da_dst,
-                    pos, n_dst, n_src, static_cast<int64_t>(H) * D, 4 * static_cast<int64_t>(H),
-                    slope, 0};
+                    pos, n_dst, n_src, n_edges, static_cast<int64_t>(H) * D,
+                    4 * static_cast<int64_t>(H), slope, 0};
   char* w = static_cast<char*>(ws);
   switch (dtype) {
     case TGX_DTYPE_F32:

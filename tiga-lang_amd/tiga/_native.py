@@ -93,6 +93,8 @@ _SIGNATURES: dict[str, list] = {
                          c_int, c_vp],
     "tgx_gat_fwd": [c_vp, c_vp, c_int, P(RowPlan), c_vp, c_vp, c_vp, c_vp, c_f32, c_vp,
                     c_vp, c_i64, c_i64, c_int, c_int, c_int, c_vp, c_vp, c_vp],
+    "tgx_gat_fwd_edges": [c_vp, c_vp, c_int, P(RowPlan), c_vp, c_vp, c_vp, c_vp, c_f32, c_vp,
+                          c_vp, c_i64, c_i64, c_i64, c_int, c_int, c_int, c_vp, c_vp, c_vp],
     "tgx_gat_bwd_workspace": [P(RowPlan), P(RowPlan), c_i64, c_int, c_int, c_int, c_int,
                               P(c_size)],
     "tgx_gat_bwd": [c_vp, c_vp, c_int, P(RowPlan), c_vp, c_vp, c_vp, c_vp, P(RowPlan), c_vp,

@@ -205,10 +205,10 @@ class GatFunction(torch.autograd.Function):
         plan = graph._row_plan()
         partial = _partial(plan, 2 * H * D + 3 * H if pos is not None else H * D + 2 * H,
                            hs.device)
-        _native.call("tgx_gat_fwd", row_ptr.data_ptr(), col_idx.data_ptr(),
+        _native.call("tgx_gat_fwd_edges", row_ptr.data_ptr(), col_idx.data_ptr(),
                      _native.idx_bits(row_ptr), plan.ref, hs.data_ptr(), hd.data_ptr(),
                      asc.data_ptr(), adc.data_ptr(), float(slope), out.data_ptr(),
-                     ns.data_ptr(), n_dst, n_src, H, D, _VALUE_DTYPES[hs.dtype], _p(partial),
+                     ns.data_ptr(), n_dst, n_src, col_idx.numel(), H, D, _VALUE_DTYPES[hs.dtype], _p(partial),
                      _p(pos), _native.stream_of(hs))
         ctx.graph = graph
         ctx.slope = float(slope)
