@@ -343,6 +343,38 @@ def test_wide_edge_weight_gradient_without_its_workspace(monkeypatch):
     assert float((got[1] - want[1]).abs().max()) <= RTOL32 * float(want[1].abs().max())
 
 
+def test_skewed_16_bit_sums_are_no_slower_than_fp32():
+    """Rows of 0 to 512 edges, most of them short: 100 bf16 values a row take
+    no longer than 100 fp32 ones (four rows to a wave, its long ones one after
+    the other, took half as long again)."""
+    print("skewed bf16 sums", flush=True)
+    n = 16_384
+    g = torch.Generator(device=DEV).manual_seed(0)
+    deg = (512 * torch.rand(n, device=DEV, generator=g) ** 8).long()
+    row_ptr = torch.zeros(n + 1, dtype=torch.int64, device=DEV)
+    row_ptr[1:] = torch.cumsum(deg, 0)
+    E = int(row_ptr[-1])
+    graph = tg.Graph.from_csr(row_ptr, torch.randint(0, n, (E,), device=DEV, generator=g),
+                              num_src=n)
+    from tiga._ops import CsrSumFunction
+
+    w = torch.rand(E, device=DEV, generator=g)
+    x = torch.randn(n, 100, device=DEV, generator=g)
+    best = {}
+    for dtype in (torch.float32, torch.bfloat16) * 2:
+        xd = x.to(dtype)
+        for _ in range(10):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            for _ in range(20):   # (the host runs ahead: the kernels' time)
+                CsrSumFunction.apply(xd, w, graph)
+            end.record()
+            end.synchronize()
+            best[dtype] = min(best.get(dtype, 1e9), start.elapsed_time(end) / 20)
+    print("   ms:", best, flush=True)
+    assert best[torch.bfloat16] <= 1.1 * best[torch.float32]
+
+
 # ---- GAT additive ----------------------------------------------------------
 
 class GAT(tg.MessagePassing):

@@ -20,8 +20,7 @@
 // (Infinity Cache or HBM alike, 64 or 128 bytes of a line alike), 7 TB/s of
 // whole lines, and a random row costs the lines it touches.  100,000 rows of
 // 16 neighbours, 64 floats: 57 us for 3.2 M lines; 200,000 rows of 12
-// neighbours, 100 bf16: 178 us with one row per wave and 8-byte loads, 116 us
-// for 6.1 M lines now.  (Column tiles of 128 bytes, each XCD's L2 holding one
+// neighbours, 100 bf16: 178 us with 8-byte loads, 112 us for 6.1 M lines now.  (Column tiles of 128 bytes, each XCD's L2 holding one
 // of a 20,000 x 500 table, measured slower than whole rows, 60 against 52 us:
 // the edges are then walked 16 times.)
 #include <hip/hip_runtime.h>
@@ -329,7 +328,7 @@ __global__ __launch_bounds__(kTaskBlock) void sum_rows_kernel(SumArgs<I, DT> a) 
                              dw_stage[threadIdx.x / kWave]);
 }
 
-// Narrow tiles (G <= 16 lanes per edge): the wave splits into 64 / SLOT lane
+// Narrow tiles (G <= 8 lanes per edge): the wave splits into 64 / SLOT lane
 // slots of SLOT lanes, each taking P rows of the wave bin, so a wave's fixed
 // cost (task decode, the dependent row_ptr -> col -> gather chain) covers
 // (64 / SLOT) P rows, and the loads of a slot's P rows are in flight
@@ -505,23 +504,25 @@ template <typename I, int DT, int VEC, int G>
 void launch_sum(const SumArgs<I, DT>& a, int tiles, hipStream_t s) {
   constexpr int U = (kWave / G) >= 16 ? 1 : (16 / (kWave / G) < 8 ? 16 / (kWave / G) : 8);
   const PlanView& p = a.plan;
-  // Rows of up to 8 lanes share a wave, and so do 16-lane rows of 16-bit
-  // values: they are shorter in time, so a row's fixed cost weighs more
-  // (12-edge rows of 100 bf16: 178 us a row per wave, 156 two, 116 four; 16
-  // lanes of fp32, 16-edge rows: 57, 58 and 61 us).
-  if constexpr (G <= 8 || (G == 16 && DT != TGX_DTYPE_F32)) {
+  // Rows of up to 8 lanes share a wave: they are short in time, so a row's fixed
+  // cost weighs more.  Not rows of 16 lanes: four to a wave gain nothing on even
+  // degrees (bf16 F = 100, 12-edge rows 112 us, 111 one a wave) and a wave of
+  // several long rows ends late (R-MAT, 262,144 rows of 16 edges 188 against 132,
+  // 16,384 rows of 32 edges 68 against 33).
+  if constexpr (G <= 8) {
     // One lane per edge: 16-lane slots of 2 rows each, 8 rows per wave (the
     // reference's F = 1 case, 131072 rows of 16 edges: 0.0254 ms with 32-lane
     // slots of 2 rows, 0.0182 ms with these).  2 to 8 lanes: 32-lane slots of
-    // one row (two rows per wave measured 5% faster than four on 8-wide rows).
-    constexpr int SLOT = G == 1 || G == 16 ? 16 : 32;
+    // one row (two rows per wave measured 5% faster than four on 8-wide rows;
+    // 8 lanes, bf16 F = 64, 16-edge rows 36 us against 43 one a wave, though
+    // R-MAT 111 against 102).
+    constexpr int SLOT = G == 1 ? 16 : 32;
     constexpr int P = G == 1 ? 2 : 1;
     constexpr int NS = kWave / SLOT;
-    constexpr int US = G < 8 ? G : 8;
     const int64_t waves = p.n_chunks + (p.n_wave + NS * P - 1) / (NS * P) +
                           (p.n_empty + kEmptyPerWave - 1) / kEmptyPerWave;
-    const auto k = a.self_x ? sum_pairs_kernel<I, DT, VEC, G, U, SLOT, P, US, true>
-                            : sum_pairs_kernel<I, DT, VEC, G, U, SLOT, P, US, false>;
+    const auto k = a.self_x ? sum_pairs_kernel<I, DT, VEC, G, U, SLOT, P, G, true>
+                            : sum_pairs_kernel<I, DT, VEC, G, U, SLOT, P, G, false>;
     k<<<static_cast<unsigned>(ceil_div(waves, kWavesPerBlock)), kTaskBlock, 0, s>>>(a);
   } else {
     const dim3 grid(static_cast<unsigned>(ceil_div(plan_waves(p), kWavesPerBlock)),
