@@ -14,6 +14,7 @@ import torch
 from torch import nn
 
 import tiga as tg
+from tiga import _native
 from oracle import ref
 
 pytestmark = pytest.mark.gpu
@@ -549,3 +550,19 @@ def test_projected_hub_costs_no_more_than_its_edges():
         times.append(best)
     print("   backward without and with a hub, ms:", times, flush=True)
     assert times[1] <= 2 * times[0]
+
+
+def test_uncovered_chains_are_told_apart_without_an_exception(monkeypatch):
+    """A two-layer chain that the per-row kernels do not cover (17 hidden
+    units) goes to the per-edge ones on a status, not on an error per call."""
+    print("uncovered chain", flush=True)
+    raised = []
+    raise_status = _native.raise_status
+    monkeypatch.setattr(_native, "raise_status",
+                        lambda *args: (raised.append(args), raise_status(*args)))
+    rp, col = random_graph(50, 60, 9, 3)
+    graph = tg.Graph.from_csr(rp, col, num_src=60)
+    net = nn.Sequential(nn.Linear(16, 17), nn.ReLU(), nn.Linear(17, 1)).to(DEV)
+    x, y = torch.randn(60, 8, device=DEV), torch.randn(50, 8, device=DEV)
+    out = ProjectedScore(net, ("x", "y"), "x")(graph=graph, src={"x": x}, dst={"y": y}, edge={})
+    assert out.shape == (50, 8) and not raised

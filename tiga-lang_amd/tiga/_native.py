@@ -228,12 +228,24 @@ def call(name: str, *args) -> None:
         raise_status(name, status)
 
 
+def covered(name: str, *args) -> bool:
+    """Whether entry point `name` takes these arguments: False where it answers
+    TGX_UNSUPPORTED, for callers that then go another way."""
+    status = getattr(lib(), name)(*args)
+    if status not in (0, _UNSUPPORTED):
+        raise_status(name, status)
+    return status == 0
+
+
+_UNSUPPORTED = 2
+
+
 def raise_status(name: str, status: int) -> None:
     """Raise the error a nonzero status of entry point `name` stands for."""
     handle = lib()
     message = handle.tgx_last_error().decode(errors="replace")
     kind = handle.tgx_status_string(status).decode()
-    error = NotImplementedError if status == 2 else RuntimeError
+    error = NotImplementedError if status == _UNSUPPORTED else RuntimeError
     raise error(f"{name}: {kind}: {message}")
 
 

@@ -715,10 +715,8 @@ def _projected_state(graph: Graph, mlp, E: int, device) -> torch.Tensor | None:
     if mlp.n_layers != 2 or E < max(n_dst, 1):
         return None
     floats = ctypes.c_int64()
-    try:
-        _native.call("tgx_edge_mlp_projected_state", n_dst, ctypes.byref(mlp),
-                     ctypes.byref(floats))
-    except NotImplementedError:
+    if not _native.covered("tgx_edge_mlp_projected_state", n_dst, ctypes.byref(mlp),
+                           ctypes.byref(floats)):
         return None
     return torch.empty(floats.value, dtype=torch.float32, device=device)
 
