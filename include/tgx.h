@@ -629,7 +629,8 @@ int tgx_edge_mlp_scores(const void* col_dev, const int32_t* dst_index_dev, int i
  *   tgx_edge_mlp_projected_state: floats of the state buffer (16-byte
  *     aligned) the scores fill and the backward reads; TGX_UNSUPPORTED where
  *     the kernels do not cover the chain (two layers, up to 16 hidden units,
- *     functions up to TGX_ACT_MISH but TGX_ACT_HARDTANH, no LayerNorm, source
+ *     functions up to TGX_ACT_MISH but TGX_ACT_HARDTANH and a softplus whose
+ *     threshold lies beyond 1e30 / beta, no LayerNorm, source
  *     fields of up to 8 floats in all, destination fields of 1 to 16, edge
  *     fields of up to 7, at most two of a role): the caller then uses
  *     the entry points above, as it may for any chain.

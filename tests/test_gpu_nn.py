@@ -566,3 +566,32 @@ def test_uncovered_chains_are_told_apart_without_an_exception(monkeypatch):
     x, y = torch.randn(60, 8, device=DEV), torch.randn(50, 8, device=DEV)
     out = ProjectedScore(net, ("x", "y"), "x")(graph=graph, src={"x": x}, dst={"y": y}, edge={})
     assert out.shape == (50, 8) and not raised
+
+
+@pytest.mark.parametrize("hidden", [13, 16])
+@pytest.mark.parametrize("act", [nn.Softplus(), nn.Softplus(2.0, torch.inf),
+                                 nn.Softplus(0.5, 3e38), nn.Mish(), nn.SELU(), nn.Sigmoid()])
+def test_projected_padding_units(hidden, act):
+    """Units past the hidden width hold no value that reaches a score or a
+    gradient, whatever the function and its parameters (a softplus without a
+    threshold overflows where others are linear)."""
+    print("projected padding", hidden, act, flush=True)
+    torch.manual_seed(hidden)
+    rows, n_src = 60, 70
+    rp, col = random_graph(rows, n_src, 9, 3)
+    graph = tg.Graph.from_csr(rp, col, num_src=n_src)
+    net = nn.Sequential(nn.Linear(16, hidden), act, nn.Linear(hidden, 1, bias=False))
+    x, y, dout = torch.randn(n_src, 8), torch.randn(rows, 8), torch.randn(rows, 8)
+    xw, yw = (t.double().requires_grad_(True) for t in (x, y))
+    net64 = nn.Sequential(*net).double()
+    c, r = col.cpu(), torch.repeat_interleave(torch.arange(rows), rp.cpu().diff())
+    ex = net64(torch.cat([xw[c], yw[r]], 1)).squeeze(1).exp()   # (scores of order 1)
+    alpha = ex / torch.zeros(rows, dtype=torch.float64).index_add(0, r, ex)[r]
+    out64 = torch.zeros(rows, 8, dtype=torch.float64).index_add(0, r, alpha[:, None] * xw[c])
+    expect = [out64, *torch.autograd.grad(out64, [xw, yw, *net64.parameters()], dout.double())]
+    net = net64.float().to(DEV)
+    xg, yg = (t.to(DEV).requires_grad_(True) for t in (x, y))
+    out = ProjectedScore(net, ("x", "y"), "x")(graph=graph, src={"x": xg}, dst={"y": yg}, edge={})
+    got = [out, *torch.autograd.grad(out, [xg, yg, *net.parameters()], dout.to(DEV))]
+    for a, e in zip(got, expect):
+        assert rel_err(f64(a), e.detach()) <= 3e-5
