@@ -291,3 +291,20 @@ def test_coo_sources_are_moved_as_they_are(n_rows, n_edges, src_bits):
                          ws_bytes.value, _native.stream_of(dst))
             assert torch.equal(col, src[order])
             assert perm is None or torch.equal(perm.long(), order)
+
+
+def test_transpose_checks_what_a_caller_may_have_changed():
+    """destination_index() hands out the graph's cached row ids, and a graph
+    takes any integer as its source count: a transpose refuses row ids out of
+    range and counts that from_coo refuses."""
+    print("transpose checks", flush=True)
+    row_ptr = torch.tensor([0, 2, 3], device=DEV)
+    col = torch.tensor([0, 1, 1], device=DEV)
+    graph = tg.Graph.from_csr(row_ptr, col, num_src=2)
+    graph.destination_index()[1] = 2**40
+    with pytest.raises(ValueError, match="src contains an out-of-range"):
+        graph.transpose()
+    with pytest.raises(ValueError, match="num_dst must be a non-negative integer"):
+        tg.Graph.from_csr(row_ptr, col, num_src=np.int64(2)).transpose()
+    assert tg.Graph.from_csr(row_ptr, col, num_src=2).transpose().resolve_csr()[1].tolist() == \
+        [0, 0, 1]

@@ -314,16 +314,16 @@ class Graph:
             num_src = int(src.max().item()) + 1 if src.numel() else 0
         if num_dst is None:
             num_dst = int(dst.max().item()) + 1 if dst.numel() else 0
-        if not isinstance(num_src, int) or num_src < 0:
-            raise ValueError("num_src must be a non-negative integer")
-        if not isinstance(num_dst, int) or num_dst < 0:
-            raise ValueError("num_dst must be a non-negative integer")
         return cls._from_coo(src, dst, num_src, num_dst)
 
     @classmethod
     def _from_coo(cls, src, dst, num_src: int, num_dst: int, src_known: bool = False) -> "Graph":
-        """from_coo on checked shapes and counts; src_known: every source is
-        in range by construction (the row ids of a transpose)."""
+        """from_coo on checked shapes; src_known: every source is in range by
+        construction (the row ids of a transpose, formed for it)."""
+        if not isinstance(num_src, int) or num_src < 0:
+            raise ValueError("num_src must be a non-negative integer")
+        if not isinstance(num_dst, int) or num_dst < 0:
+            raise ValueError("num_dst must be a non-negative integer")
         if src.numel():
             if src.is_cuda:
                 *src_bad, dst_bad = _indices_out_of_range(
@@ -532,8 +532,9 @@ class Graph:
             self._destination_index_cache = destination
         if destination.shape != col_idx.shape:
             raise ValueError("src and dst must have identical shapes")
+        # (Cached row ids have been in the caller's hands: checked as before.)
         return self._from_coo(destination, col_idx, self._schema.num_dst, self._schema.num_src,
-                              src_known=True)
+                              src_known=cached is None)
 
     def destination_index(self, row_ptr: torch.Tensor | None = None) -> torch.Tensor:
         if row_ptr is None and self._destination_index_cache is not None:
