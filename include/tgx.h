@@ -623,9 +623,10 @@ int tgx_edge_mlp_scores(const void* col_dev, const int32_t* dst_index_dev, int i
                         void* stream);
 
 /* Two-layer networks over destination fields with the first layer's destination
- * columns applied once per row instead of once per edge: scores as tgx_edge_mlp_scores gives them, up to fp32 rounding, and
- * the attention backward as tgx_edge_mlp_attention_backward's, except that
- * destination fields' gradients come back per row.
+ * columns applied once per row instead of once per edge: scores as
+ * tgx_edge_mlp_scores gives them, up to fp32 rounding, and the attention
+ * backward as tgx_edge_mlp_attention_backward's, except that destination
+ * fields' gradients come back per row.
  *   tgx_edge_mlp_projected_state: floats of the state buffer (16-byte
  *     aligned) the scores fill and the backward reads; TGX_UNSUPPORTED where
  *     the kernels do not cover the chain (two layers, up to 16 hidden units,

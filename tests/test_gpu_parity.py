@@ -236,10 +236,9 @@ def test_sum_of_edge_field_per_row(F_, idx):
     assert rel_err(out.cpu(), ref.sum_fwd(rp, np.arange(E), x)) <= RTOL32
 
 
-# Widths at the edges of a lane's values (4 fp32, 8 16-bit) and of the lane
-# groups, rows aligned to their elements only; tables one L2 holds whole (900
-# source rows of few values), a column tile at a time (9,000 rows of 260 or
-# more values), and not at all (70,000 destination rows: the backward's).
+# Widths at the edges of a lane's values (4 fp32, 8 16-bit), of the lane groups
+# and of the feature tiles (256 fp32, 512 16-bit), rows aligned to their elements
+# only; tables that one XCD's L2 holds (900 and 3,000 rows) and that none does.
 @pytest.mark.parametrize("n_dst,n_src,F_", [
     *[(1500, 900, f) for f in (1, 3, 4, 5, 7, 8, 9, 31, 33, 63, 65, 127, 129, 255, 257)],
     (9000, 9000, 260), (9000, 8000, 301), (6000, 40000, 517), (5000, 3000, 1030),
