@@ -43,7 +43,7 @@ BF16_PEAK_TFLOPS = 2500.0   # MI355X dense bf16 (and fp16) MFMA
 
 
 def measured_traffic(config, kernel):
-    """L2-to-memory bytes per launch of `kernel` (or the sum over a
+    """L2-to-memory bytes per step of `kernel` (or the sum over a
     "+"-joined list of kernels that run once per step each) measured by
     rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE (scaled by the copy calibration)
     and recorded in profiles/traffic.json; None when any is unrecorded.

@@ -80,8 +80,9 @@ constexpr int VBN = 64;    // keys per iteration
 // first part of each row.
 constexpr int TPAD = 144;
 // The forward's, by head dim, and the workgroups per CU its registers are held
-// to: 160 and 96 B rows are as free of conflicts (eight rows fall on distinct
-// banks), and with 288 B ones the double-buffered K and V tiles left room for
+// to: 160 B rows are as free of conflicts (eight rows fall on distinct banks), 96
+// B ones nearly (2.7M conflict cycles a launch of the 96 us below, some 4 us of
+// it), and with 288 B ones the double-buffered K and V tiles left room for
 // two workgroups per CU at every D.  24 causal sequences of 500 to 2000
 // tokens: D = 64, 12 heads 125 -> 110 us, D = 32, 16 heads 118 -> 96 us.  (The
 // backward's tiles are single-buffered and not bound by LDS capacity: the same
