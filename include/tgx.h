@@ -114,7 +114,7 @@ int tgx_coo_to_csr(const void* src_dev, int src_bits, const void* dst_dev,
                    void* workspace_dev, size_t workspace_bytes, void* stream);
 
 /* tgx_coo_to_csr where every src is known to lie in [0, n_src): 64-bit sources
- * of n_src <= 2^31 then move as 32-bit values through the sort (a source
+ * of 0 < n_src <= 2^31 then move as 32-bit values through the sort (a source
  * outside would be cut), instead of being gathered after it.  The workspace is
  * tgx_coo_to_csr_workspace's. */
 int tgx_coo_to_csr_in_range(const void* src_dev, int src_bits, const void* dst_dev,
@@ -631,7 +631,7 @@ int tgx_edge_mlp_scores(const void* col_dev, const int32_t* dst_index_dev, int i
  *     aligned) the scores fill and the backward reads; TGX_UNSUPPORTED where
  *     the kernels do not cover the chain (two layers, up to 16 hidden units,
  *     functions up to TGX_ACT_MISH but TGX_ACT_HARDTANH and a softplus whose
- *     threshold lies beyond 1e30 / beta, no LayerNorm, source
+ *     threshold lies beyond 1e30 beta, no LayerNorm, source
  *     fields of up to 8 floats in all, destination fields of 1 to 16, edge
  *     fields of up to 7, at most two of a role): the caller then uses
  *     the entry points above, as it may for any chain.

@@ -1143,16 +1143,16 @@ extern "C" int tgx_gat_fwd_edges(const void* row_ptr, const void* col, int idx_b
   switch (dtype) {
     case TGX_DTYPE_F32:
       return gat_fwd_dtype<TGX_DTYPE_F32>(row_ptr, col, idx_bits, plan, h_src, h_dst, a_src,
-                                          a_dst, slope, out, ns, n_dst, n_src, n_edges, H, D, partial,
-                                          pos, s);
+                                          a_dst, slope, out, ns, n_dst, n_src, n_edges, H, D,
+                                          partial, pos, s);
     case TGX_DTYPE_BF16:
       return gat_fwd_dtype<TGX_DTYPE_BF16>(row_ptr, col, idx_bits, plan, h_src, h_dst, a_src,
-                                           a_dst, slope, out, ns, n_dst, n_src, n_edges, H, D, partial,
-                                          pos, s);
+                                           a_dst, slope, out, ns, n_dst, n_src, n_edges, H, D,
+                                          partial, pos, s);
     default:
       return gat_fwd_dtype<TGX_DTYPE_F16>(row_ptr, col, idx_bits, plan, h_src, h_dst, a_src,
-                                          a_dst, slope, out, ns, n_dst, n_src, n_edges, H, D, partial,
-                                          pos, s);
+                                          a_dst, slope, out, ns, n_dst, n_src, n_edges, H, D,
+                                          partial, pos, s);
   }
 }
 

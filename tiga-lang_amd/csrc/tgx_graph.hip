@@ -1174,8 +1174,8 @@ extern "C" int tgx_coo_to_csr_in_range(const void* src, int src_bits, const void
                                        int64_t n_edges, void* row_ptr, void* col, int32_t* perm,
                                        void* ws, size_t ws_bytes, void* stream) {
   TGX_REQUIRE(n_src >= 0, "negative size");
-  return coo_checked(src, src_bits, dst, dst_bits, n_src <= (int64_t{1} << 31), n_dst, n_edges,
-                     row_ptr, col, perm, ws, ws_bytes, stream);
+  return coo_checked(src, src_bits, dst, dst_bits, n_src > 0 && n_src <= (int64_t{1} << 31),
+                     n_dst, n_edges, row_ptr, col, perm, ws, ws_bytes, stream);
 }
 
 extern "C" int tgx_varlen_csr_workspace(int64_t n_seq, size_t* bytes) {

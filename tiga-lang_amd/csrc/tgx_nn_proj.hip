@@ -725,7 +725,7 @@ int proj_view(const tgx_edge_mlp* m, ProjView* out) {
   // beyond it takes the exponential there.)
   if (m->act[0] == TGX_ACT_SOFTPLUS && m->act_param[0] > 0.f &&
       !(m->act_param[0] * kNoUnit > m->act_param2[0]))
-    return unsupported("softplus with a threshold below 1e30 / beta");
+    return unsupported("softplus with a threshold below 1e30 beta");
   TGX_REQUIRE(m->width == 16 || m->width == 24 || m->width == 32, "bad padded width");
   TGX_REQUIRE(m->n_segments >= 1 && m->n_segments <= kMaxSegments, "bad segment count");
   v.hidden = m->out_width[0] ? m->out_width[0] : m->width;

@@ -20,9 +20,10 @@
 // (Infinity Cache or HBM alike, 64 or 128 bytes of a line alike), 7 TB/s of
 // whole lines, and a random row costs the lines it touches.  100,000 rows of
 // 16 neighbours, 64 floats: 57 us for 3.2 M lines; 200,000 rows of 12
-// neighbours, 100 bf16: 178 us with 8-byte loads, 112 us for 6.1 M lines now.  (Column tiles of 128 bytes, each XCD's L2 holding one
-// of a 20,000 x 500 table, measured slower than whole rows, 60 against 52 us:
-// the edges are then walked 16 times.)
+// neighbours, 100 bf16: 178 us with 8-byte loads, 112 us for 6.1 M lines now.
+// (Column tiles of 128 bytes, each XCD's L2 holding one of a 20,000 x 500 table,
+// measured slower than whole rows, 60 against 52 us: the edges are then walked 16
+// times.)
 #include <hip/hip_runtime.h>
 
 #include <climits>
